@@ -20,7 +20,9 @@
 extern "C" int p3e_launch_step(const void *table, const void *work, int nwork, int prec, size_t lds,
                                unsigned int grid, hipStream_t st);
 extern "C" int p3e_step_occupancy(int prec, size_t lds);
-extern "C" int p3e_launch_group(int kind, int M, const void *tab, const void *start, int n, int prec, size_t lds,
+extern "C" int p3e_launch_pass(const p3e::PassArgs *a, int prec, size_t lds_bytes, int threads,
+                               unsigned int nblocks, hipStream_t st);
+extern "C" int p3e_launch_group(int kind, int M, const p3e::PassArgs *first, const void *tab, const void *start, int n, int prec, size_t lds,
                                 int threads, unsigned int nblocks, hipStream_t st);
 
 namespace p3e {
@@ -139,11 +141,13 @@ static std::string tune_key(int prec, const PassDesc &pd) {
   const PassArgs &a = pd.args;
   char k[256];
   snprintf(k, sizeof(k), "gfx950:p%d:c%d:k%d:N%d:W%d:L%d:o%d%d:e%d:m%d", prec, a.cls, a.r2r_kind, a.N, a.W, a.L,
-           a.load_order, a.store_order, a.ne, a.mid);
+           a.load_order, a.store_order, a.ne, a.mid + (a.mid && a.tw_in_lds ? 2 : 0));
   return k;
 }
 
-// Time one candidate: all tiles of the pass through the step kernel.
+// Time one candidate: all tiles of the pass through the step kernel, or, for
+// a single-buffer pass planned for its own kernel (a grouped batch), through
+// that.
 static float time_candidate(int prec, PassDesc &pd, void *din, void *dout, PassArgs *d_tab, WorkItem *d_work,
                             int maxwork, hipStream_t st) {
   PassArgs a = pd.args;
@@ -162,7 +166,9 @@ static float time_candidate(int prec, PassDesc &pd, void *din, void *dout, PassA
   float best = 1e30f;
   for (int rep = 0; rep < 4; rep++) {
     (void)hipEventRecord(e0, st);
-    int rc = p3e_launch_step(d_tab, d_work, nw, prec, pd.lds_bytes, grid, st);
+    int rc = pd.args.mid && pd.args.tw_in_lds
+                 ? p3e_launch_pass(&a, prec, pd.lds_bytes, pd.threads, (unsigned int)nw, st)
+                 : p3e_launch_step(d_tab, d_work, nw, prec, pd.lds_bytes, grid, st);
     (void)hipEventRecord(e1, st);
     (void)hipEventSynchronize(e1);
     if (rc) {
@@ -266,11 +272,18 @@ static bool plan_items(BatchPlan *b, const OpSpec ops[3], const int order[3], in
 }
 
 // Grouped kernel of a standalone pass: 1 power-of-two, 2 single-buffer
-// without an odd prime above 5, 0 none.
+// without a prime radix above 16, 0 none.
 static int group_kind(const PassDesc &pd) {
   if (pd.args.fast) return 1;
-  if (pd.args.mid && pd.args.mid_prime == 0) return 2;
+  if (pd.args.mid && pd.args.mid_prime <= 16) return 2;
   return 0;
+}
+
+// What the passes of one grouped launch share: the length of a power-of-two
+// kernel, the class and routes of a single-buffer one.
+static int group_key(const PassArgs &a) {
+  if (a.fast) return a.M;
+  return ((a.cls * 2 + a.bluestein) * 2 + a.direct_in) * 2 + a.direct_out;
 }
 
 static bool build_groups(BatchPlan *b) {
@@ -283,7 +296,7 @@ static bool build_groups(BatchPlan *b) {
     for (int i = 0; i < b->nitems; i++) {
       const PassDesc &pd = b->chains[i].passes[s];
       const int kind = group_kind(pd);
-      by_kernel[{kind, kind == 1 ? pd.args.M : 0}].push_back(i);
+      by_kernel[{kind, group_key(pd.args)}].push_back(i);
     }
     for (auto &kv : by_kernel) {
       BatchGroup g;
@@ -322,7 +335,7 @@ static bool build_groups(BatchPlan *b) {
       b->owned.push_back(g.d_start);
       b->groups[s].push_back(g);
       snprintf(buf, sizeof(buf), "%sstage %d %s%d: %d items, %u tiles, %d threads, LDS %zu B",
-               b->desc.empty() ? "" : " | ", s, g.kind == 1 ? "pow2 M=" : "mid", g.kind == 1 ? g.M : 0, g.n,
+               b->desc.empty() ? "" : " | ", s, g.kind == 1 ? "pow2 M=" : "mid ", g.M, g.n,
                g.nblocks, g.threads, g.lds);
       b->desc += buf;
     }
@@ -427,12 +440,15 @@ BatchPlan *batch_create(int prec, int nitems, const OpSpec ops[3], const int ord
         batch_destroy(b);
         return nullptr;
       }
-      if (tune && !b->grouped) tune_pass(prec, pd, st, b->owned);
+      if (tune) tune_pass(prec, pd, st, b->owned);
       if (!tables_ready(pd)) {
         set_error("batch: tuning lost a constant table");
         batch_destroy(b);
         return nullptr;
       }
+      // the direct routes of real lines depend on the alignment of each
+      // exec's arrays; a grouped launch's kernel is chosen once
+      if (pd.args.mid && pd.args.cls != CLS_C2C) pd.args.direct_in = pd.args.direct_out = 0;
     }
   // scratch: worst case over the in != out and in == out assignments
   b->scratch_off.resize(2 * nitems);
@@ -519,7 +535,7 @@ static int batch_launch(BatchPlan *b, hipStream_t st) {
       }
       for (const BatchGroup &g : gs) {
         hipStream_t gst = g.q == 0 ? st : b->side[g.q - 1];
-        const int rc = p3e_launch_group(g.kind, g.M, b->d_table + g.tab0, g.d_start, g.n, b->prec, g.lds, g.threads,
+        const int rc = p3e_launch_group(g.kind, g.M, &b->table[g.tab0], b->d_table + g.tab0, g.d_start, g.n, b->prec, g.lds, g.threads,
                                         g.nblocks, gst);
         if (rc) {
           set_error("batch group launch failed: %s", hipGetErrorString((hipError_t)rc));

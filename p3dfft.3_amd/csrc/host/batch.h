@@ -10,8 +10,8 @@
 namespace p3e {
 
 // A grouped launch of a batch stage: the same pass kernel (power-of-two of
-// complex length M, kind 1; single-buffer without an odd prime above 5,
-// kind 2) over n items whose PassArgs are table entries tab0 .. tab0+n-1.
+// complex length M, kind 1; single-buffer without a prime radix above
+// 16, of one class and route, kind 2) over n items whose PassArgs are table entries tab0 .. tab0+n-1.
 struct BatchGroup {
   int kind, M;
   int threads;             // the largest of the items'
@@ -69,7 +69,7 @@ struct BatchPlan {
 };
 
 // ops/order as for plan_create; in[i]/out[i] are the layouts of item i.
-// tune: run the autotuner for the generic-path passes (results cached).
+// tune: run the autotuner for the passes without a compile-time length (results cached).
 BatchPlan *batch_create(int prec, int nitems, const OpSpec ops[3], const int order[3], const Layout *in,
                         const Layout *out, bool tune);
 // in[i]/out[i]: device pointers of item i.  sync: wait for completion.

@@ -215,80 +215,298 @@ static bool is_pow2(int n) { return n > 0 && (n & (n - 1)) == 0; }
 
 static bool radix_supported(int r);
 
-static bool mid_base_radix(int r) { return r == 2 || r == 3 || r == 4 || r == 5 || r == 8 || r == 16; }
+// Radices of the single-buffer kernel without an odd prime above 16, and of
+// its kernels with one (fft_mid.h, mid_fft).
+static bool mid_base_radix(int r, int prime = 0) {
+  return (r >= 2 && r <= 10) || r == 12 || r == 16 || (prime == 0 && (r == 11 || (r >= 13 && r <= 15)));
+}
 
 // Largest odd prime radix of the single-buffer kernels: 47 in FP32; 29 in
 // FP64, where the registers of a larger butterfly (two doubles per complex
 // value) exceed the 256 VGPRs of a wave and would spill.
 static int mid_max_prime(int prec) { return prec == 8 ? 29 : 47; }
 
-// The odd prime radix of a radix list that the single-buffer path takes: 0
-// if every radix is 2, 3, 4, 5, 8 or 16, the prime if there is one distinct
-// other radix and it is a prime from 7 to mid_max_prime(prec), -1 otherwise.
-static int mid_prime_of(const int *rad, int nrad, int prec) {
-  int p = 0;
-  for (int i = 0; i < nrad; i++) {
-    const int r = rad[i];
-    if (mid_base_radix(r)) continue;
-    if (r < 7 || r > mid_max_prime(prec) || (p != 0 && r != p)) return -1;
-    for (int q = 3; q * q <= r; q += 2)
-      if (r % q == 0) return -1;
-    p = r;
+// The odd prime radix P above 16 of a length that the single-buffer path
+// takes: 0 if its prime factors are all at most 13, the prime if exactly one
+// factor is a larger prime up to mid_max_prime(prec), -1 otherwise.
+// *named: the length's only distinct prime factor above 5, or 0.
+static int mid_prime_of(int n, int prec, int *named) {
+  int p = 0, m = n, only = 0, distinct = 0;
+  for (int q = 2; q <= m; q++) {
+    int e = 0;
+    while (m % q == 0) {
+      m /= q;
+      e++;
+    }
+    if (!e) continue;
+    if (q > 5) {
+      only = q;
+      distinct++;
+    }
+    if (q <= 13) continue;
+    if (p || e > 1 || q > mid_max_prime(prec)) return -1;
+    p = q;
   }
+  if (named) *named = distinct == 1 ? only : 0;
   return p;
 }
 
-// Switch an already described generic pass to the single-buffer mixed-radix
-// path (fft_mid.h) when every radix of the work length (the Bluestein length
-// for a large prime) is 2, 3, 4, 5, 8 or 16, plus — for a standalone pass
-// kernel, not the batch kernel — at most one distinct odd prime 7..47 (its
-// own kernel instantiation).  Other passes stay on the two-buffer generic
-// path.  Tile: B lines with B * L <= 16 threads' worth of elements, as
-// large as LDS and the workgroup size (512 threads, or the batch kernel's)
-// allow; the twiddles go to LDS after the lines when they fit.
-static void setup_mid(int prec, const OpSpec &op, PassDesc &ps, int batch_threads) {
-  PassArgs &a = ps.args;
-  if (op.cls == CLS_EMPTY || a.nrad < 1) return;
-  const int prime = mid_prime_of(a.radix, a.nrad, prec);
-  if (prime < 0 || (prime > 0 && batch_threads > 0)) return;
-  const int L = a.L;
-  const long maxth = batch_threads > 0 ? batch_threads : P3E_MID_THREADS(prec, prime);
-  const size_t esz = 2 * (size_t)prec;
-  const size_t per_line = (size_t)a.lpad * esz;
-  size_t twl = batch_threads > 0 ? 0 : ps.tw.size() * esz;
-  if (per_line + twl > LDS_MAX) twl = 0;
-  // R2C / C2R: two real lines per LDS line (fft_mid.h, pair_load)
-  const bool pair = op.cls == CLS_R2C || op.cls == CLS_C2R;
-  auto lines = [&](int b) { return pair ? (b + 1) / 2 : b; };
-  int B = 1;
-  const int Bmax = std::min(pair ? 64 : 32, next_pow2(a.ne));
-  const long E = P3E_MID_E;
-  while (B * 2 <= Bmax && per_line * lines(B * 2) + twl <= P3E_MID_LDS && (long)lines(B * 2) * L <= E * maxth)
-    B *= 2;
-  if (per_line * lines(B) + twl > LDS_MAX || (long)lines(B) * L > E * maxth) return;
-  int th = (int)(((long)lines(B) * L + E - 1) / E);
-  th = std::max(64, (th + 63) & ~63);
-  if (th > maxth) return;
-  // the kernel addresses a tile's elements with 32-bit byte offsets from
-  // the tile's first element (below 2^31 on both sides)
-  const double in_esz = (double)prec * (a.in_cplx ? 2 : 1), out_esz = (double)prec * (a.out_cplx ? 2 : 1);
-  if (((double)a.nin * a.is_d + (double)B * a.is_e + 1) * in_esz >= 2147483648.0 ||
-      ((double)a.nout * a.os_d + (double)B * a.os_e + 1) * out_esz >= 2147483648.0)
+// Cost of a radix-R pass per element, in instructions: LDS read and write,
+// twiddle and barriers, plus the butterfly.
+static double mid_radix_cost(int R) {
+  switch (R) {
+    case 2: return 14;
+    case 3: return 18;
+    case 4: return 16;
+    case 5: return 20;
+    case 6: return 19;
+    case 7: return 22;
+    case 8: return 19;
+    case 9: return 23;
+    case 10: return 22;
+    case 11: return 27;
+    case 12: return 21;
+    case 13: return 29;
+    case 14: return 24;
+    case 15: return 26;
+    case 16: return 22;
+  }
+  return 16 + 1.2 * R;
+}
+
+// Threads per LDS line of a radix sequence: every pass has at most
+// mid_butterflies(R) butterflies per thread.
+static int mid_line_threads(int L, const int *rad, int nrad) {
+  int t = 1;
+  for (int i = 0; i < nrad; i++) {
+    const int nb = mid_butterflies(rad[i]);
+    t = std::max(t, (L / rad[i] + nb - 1) / nb);
+  }
+  return t;
+}
+
+// Cheapest radix sequence of length L = prime x (a product of base radices):
+// the passes' cost per element, times the threads per line over the ideal
+// L / 20 to the power 1/4 (a sequence whose passes leave many threads idle
+// pays for their registers, not for their work).
+static void mid_search(int L, int rest, int prime, int maxr, std::vector<int> &cur, double cost, double *best,
+                       std::vector<int> *out) {
+  if (rest == 1) {
+    const double t = mid_line_threads(L, cur.data(), (int)cur.size());
+    const double c = cost * pow(t * 20.0 / L, 0.25);
+    if (c < *best) {
+      *best = c;
+      *out = cur;
+    }
     return;
-  a.mid = 1;
-  a.mid_prime = prime;
-  a.pair = pair;
-  a.tw_in_lds = twl > 0;
-  a.ntw = (int)ps.tw.size();
-  a.B = B;
-  a.logB = 0;
-  while ((1 << a.logB) < B) a.logB++;
-  a.ntile_e = (a.ne + B - 1) / B;
+  }
+  if (cost >= *best || cur.size() >= P3E_MAX_RADIX_PASSES) return;
+  for (int r = std::min(maxr, 16); r >= 2; r--) {
+    if (rest % r || !mid_base_radix(r, prime)) continue;
+    cur.push_back(r);
+    mid_search(L, rest / r, prime, r, cur, cost + mid_radix_cost(r), best, out);
+    cur.pop_back();
+  }
+}
+
+// Radix sequence of work length L (prime: its prime radix above 16 or 0),
+// larger radices first; returns the cost per element.
+static double mid_radices(int L, int prime, std::vector<int> &rad) {
+  std::vector<int> cur;
+  double best = 1e30, c0 = 0;
+  rad.clear();
+  if (prime) {
+    cur.push_back(prime);
+    c0 = mid_radix_cost(prime);
+  }
+  mid_search(L, prime ? L / prime : L, prime, 16, cur, c0, &best, &rad);
+  return best;
+}
+
+// Twiddles of the passes after the first, pass by pass (MPass::tw).
+static void mid_twiddles(const int *rad, int nrad, std::vector<cld> &tw) {
+  tw.clear();
+  long long Ns = 1;
+  for (int i = 0; i < nrad; i++) {
+    const int R = rad[i];
+    if (Ns > 1)
+      for (long long k = 0; k < Ns; k++)
+        for (int r = 1; r < R; r++) tw.push_back(expi_pi(-2LL * k * r, Ns * R));
+    Ns *= R;
+  }
+  if (tw.empty()) tw.push_back(cld(1, 0));
+}
+
+// Unnormalized DFT (sign -1) of any length in long double, by its smallest
+// prime factor.  Plan-time only: the spectrum of the Bluestein chirp.
+static void host_fft(std::vector<cld> &a) {
+  const int n = (int)a.size();
+  int p = 2;
+  while (p * p <= n && n % p) p++;
+  if (n % p) p = n;
+  if (n <= 1) return;
+  const int m = n / p;
+  std::vector<std::vector<cld>> sub(p, std::vector<cld>(m));
+  for (int i = 0; i < n; i++) sub[i % p][i / p] = a[i];
+  if (m > 1)
+    for (auto &v : sub) host_fft(v);
+  std::vector<cld> w(n);
+  for (int t = 0; t < n; t++) w[t] = expi_pi(-2LL * t, n);
+  for (int k = 0; k < n; k++) {
+    cld s(0, 0);
+    for (int q = 0; q < p; q++) s += sub[q][k % m] * w[(size_t)((long long)q * k % n)];
+    a[k] = s;
+  }
+}
+
+// Tile geometry of a single-buffer pass whose work length, radices, and
+// tables are set: 2^lgl = nl LDS lines per tile.  false if the tile does not
+// fit the LDS, the workgroup or 32-bit offsets (the pass is then partly
+// changed: callers work on a copy).
+static bool mid_geometry(int prec, PassDesc &ps, int nl, int batch_threads) {
+  PassArgs &a = ps.args;
+  const size_t esz = 2 * (size_t)prec;
+  const long maxth = batch_threads > 0 ? batch_threads : P3E_MID_MAXTH;
+  a.lgl = 0;
+  while ((1 << a.lgl) < nl) a.lgl++;
+  a.pit = nl == 1 ? 1 : nl + 1;
+  a.B = a.pair ? 2 * nl : nl;
+  a.logB = a.pair ? a.lgl + 1 : a.lgl;
+  a.lpad = (int)(((long long)a.L * a.pit + a.B - 1) / a.B);
+  const long th = (long)nl * mid_line_threads(a.L, a.radix, a.nrad);
+  if (th > maxth) return false;
+  ps.threads = (int)th;
+  a.nthreads = (int)th;
+  a.tw_in_lds = batch_threads == 0;
+  ps.lds_bytes = (size_t)a.L * a.pit * esz + (a.tw_in_lds ? ps.tw.size() * esz : 0);
+  if (ps.lds_bytes > LDS_MAX) return false;
+  a.ntile_e = (a.ne + a.B - 1) / a.B;
   a.div_ntile = make_fastdiv((uint32_t)a.ntile_e);
-  ps.lds_bytes = per_line * lines(B) + twl;
-  ps.threads = th;
-  a.nthreads = th;
-  ps.nblocks = (unsigned int)((unsigned long long)a.ntile_e * (unsigned long long)a.nf);
+  const unsigned long long nbk = (unsigned long long)a.ntile_e * (unsigned long long)a.nf;
+  if (nbk > 0x7fffffffULL) return false;
+  ps.nblocks = (unsigned int)nbk;
+  // 32-bit byte offsets: along lines the whole tile, across lines its width
+  // (and, for a radix pass that accesses the array itself, L / R rows)
+  const double ie = (double)prec * (a.in_cplx ? 2 : 1), oe = (double)prec * (a.out_cplx ? 2 : 1);
+  const double in_w = ((double)a.B * a.is_e + 1) * ie, out_w = ((double)a.B * a.os_e + 1) * oe;
+  const double G2 = 2147483648.0;
+  if (a.is_d * ie >= G2 || a.os_d * oe >= G2) return false;
+  if (in_w + (a.load_order == ORD_LINE ? a.nin * ie : 0) >= G2) return false;
+  if (out_w + (a.store_order == ORD_LINE ? a.nout * oe : 0) >= G2) return false;
+  // (two radix passes at least: one pass accesses one side; a prime radix
+  // above 16 writes to LDS only)
+  const bool direct = a.nrad >= 2 && !a.bluestein && batch_threads == 0;
+  a.direct_in = direct && a.load_order == ORD_TILE && (a.cls == CLS_C2C || a.cls == CLS_R2C) &&
+                (double)(a.L / a.radix[0]) * a.is_d * ie + in_w < 2 * G2;
+  a.direct_out = direct && a.store_order == ORD_TILE && (a.cls == CLS_C2C || a.cls == CLS_C2R) &&
+                 a.radix[a.nrad - 1] <= 16 &&
+                 (double)(a.L / a.radix[a.nrad - 1]) * a.os_d * oe + out_w < 2 * G2;
+  // paired accesses (the launcher checks the array addresses): adjacent
+  // lines along a stride-1 e, or adjacent elements of a line along a
+  // stride-1 d
+  a.vec2 = a.vec2s = 0;
+  if (batch_threads == 0) {
+    const bool i_e = a.is_e == 1 && a.ne % 2 == 0 && a.is_d % 2 == 0 && a.is_f % 2 == 0;
+    const bool o_e = a.os_e == 1 && a.ne % 2 == 0 && a.os_d % 2 == 0 && a.os_f % 2 == 0;
+    const bool i_d = a.is_d == 1 && a.nin % 2 == 0 && a.is_e % 2 == 0 && a.is_f % 2 == 0;
+    const bool o_d = a.os_d == 1 && a.nout % 2 == 0 && a.os_e % 2 == 0 && a.os_f % 2 == 0;
+    const bool lin = a.load_order == ORD_LINE, lout = a.store_order == ORD_LINE;
+    if (a.cls == CLS_R2C) a.vec2 = lin ? i_d : i_e;
+    if (a.cls == CLS_C2C) a.vec2 = lin && i_d;
+    if (a.cls == CLS_C2R) a.vec2 = !lin && i_e;
+    if (a.cls == CLS_R2C) a.vec2s = !lout && o_e;
+    if (a.cls == CLS_C2C) a.vec2s = lout && o_d;
+    if (a.cls == CLS_C2R) a.vec2s = lout ? o_d : o_e;
+    if (a.cls == CLS_R2R && a.pair) a.vec2s = !lout && o_e;
+  }
+  a.div_pairs = make_fastdiv((uint32_t)std::max(a.cls == CLS_R2R ? a.N / 2 + 1 : a.nin / 2, 1));
+  a.div_pairs2 = make_fastdiv((uint32_t)std::max(a.nout / 2, 1));
+  return true;
+}
+
+// Switch an already described generic pass to the single-buffer mixed-radix
+// path (fft_mid.h) when its work length is a product of that path's radices
+// (a length with a larger prime factor runs Bluestein's convolution at the
+// cheapest such length of at least 2W - 1).  Other passes stay on the
+// two-buffer generic path.
+static void setup_mid(int prec, const OpSpec &op, PassDesc &ps, int batch_threads) {
+  if (op.cls == CLS_EMPTY || ps.args.nrad < 1) return;
+  PassDesc t = ps;
+  PassArgs &a = t.args;
+  const int N = a.N, kind = op.r2r_kind;
+  int named = 0, prime = -1;
+  a.dct_short = 0;
+  if (op.cls == CLS_R2R && (kind == REDFT10 || kind == RODFT10 || kind == REDFT01 || kind == RODFT01)) {
+    // the N-point form
+    prime = N >= 2 ? mid_prime_of(N, prec, &named) : -1;
+    if (batch_threads > 0 && prime > 0) prime = -1;
+    if (prime >= 0) {
+      a.dct_short = 1;
+      a.bluestein = 0;
+      a.W = a.L = N;
+      a.zero_fill = 0;
+      a.post_off = a.post_mode = 0;
+      t.chirp.clear();
+      t.chirp_hat.clear();
+      t.pre.clear();
+      t.post.clear();
+      const bool inv = kind == REDFT01 || kind == RODFT01;
+      std::vector<cld> &tab = inv ? t.pre : t.post;
+      tab.resize(N);
+      for (int q = 0; q < N; q++) tab[q] = expi_pi(inv ? q : -q, 2LL * N);  // e^{+-i pi q / 2N}
+    }
+  }
+  std::vector<int> rad;
+  if (!a.dct_short) {
+    prime = a.bluestein ? -1 : mid_prime_of(a.W, prec, &named);
+    if (batch_threads > 0 && prime > 0) return;
+    if (!a.bluestein && prime < 0) return;
+  }
+  if (a.bluestein) {
+    // every length up to the next power of two: smallest cost of both FFTs
+    const int lo = 2 * a.W - 1, hi = next_pow2(lo);
+    double best = 1e30;
+    std::vector<int> r;
+    for (int L = lo; L <= hi; L++) {
+      if (mid_prime_of(L, prec, nullptr) != 0) continue;
+      const double c = mid_radices(L, 0, r) * L;
+      if (c < best) {
+        best = c;
+        a.L = L;
+        rad = r;
+      }
+    }
+    prime = named = 0;
+    std::vector<cld> b(a.L, cld(0, 0));
+    for (int m = 0; m < a.W; m++) b[m] = std::conj(t.chirp[m]);
+    for (int m = 1; m < a.W; m++) b[a.L - m] = std::conj(t.chirp[m]);
+    host_fft(b);
+    for (int m = 0; m < a.L; m++) b[m] /= (long double)a.L;
+    t.chirp_hat = b;
+    if (op.cls != CLS_R2R) a.zero_fill = 0;
+  } else {
+    mid_radices(a.L, prime, rad);
+  }
+  if (rad.empty() || rad.size() > P3E_MAX_RADIX_PASSES) return;
+  a.nrad = (int)rad.size();
+  for (int i = 0; i < a.nrad; i++) a.radix[i] = rad[i];
+  set_radix_divs(a);
+  mid_twiddles(a.radix, a.nrad, t.tw);
+  a.ntw = (int)t.tw.size();
+  a.mid = 1;
+  a.mid_prime = batch_threads > 0 ? 0 : (prime > 0 ? prime : named);
+  a.pair = op.cls == CLS_R2C || op.cls == CLS_C2R || (op.cls == CLS_R2R && !a.in_cplx && !a.out_cplx);
+  // Tile width: rows of 128 bytes of the complex side when a side is tile
+  // order; half of it when one tile would not leave room for another
+  // workgroup on its CU
+  const bool line_both = a.load_order == ORD_LINE && a.store_order == ORD_LINE;
+  int nl = prec == 8 ? 8 : 16;
+  const int most = next_pow2(a.pair ? (a.ne + 1) / 2 : a.ne);
+  if (!line_both && a.L <= 128) nl *= 2;
+  nl = std::min(nl, most);
+  while (nl > 1 && (!mid_geometry(prec, t, nl, batch_threads) || t.lds_bytes > P3E_MID_LDS)) nl /= 2;
+  if (!mid_geometry(prec, t, nl, batch_threads)) return;
+  ps = t;
 }
 
 // Complex DCT-I of P + 1 points on the split form of the compile-time-length
@@ -575,15 +793,14 @@ bool describe_pass(int prec, int axis, const OpSpec &op, const Layout &lin, cons
   std::vector<int> rad;
   int L = W;
   if (op.cls != CLS_EMPTY) {
-    // A standalone FP32 pass takes odd primes up to 47 as radices when the
-    // single-buffer path can run the whole length (one distinct such prime,
-    // at most 16 elements per thread of 512, one padded line in LDS);
-    // otherwise primes up to 31 run as direct DFTs on the generic path, and
-    // a length with a larger prime factor uses Bluestein.
+    // A standalone pass takes the prime radices of the single-buffer path
+    // when that path can run the whole length (up to P3E_MID_MAXTH threads
+    // of one butterfly of the prime, one line in LDS); otherwise primes up
+    // to 31 run as direct DFTs on the generic path, and a length with a
+    // larger prime factor uses Bluestein.
     bool ok = false;
-    if (batch_threads == 0 && factor(W, rad, mid_max_prime(prec)) &&
-        mid_prime_of(rad.data(), (int)rad.size(), prec) > 31 &&
-        W <= P3E_MID_E * 512 && (size_t)generic_pitch(W) * 2 * (size_t)prec <= LDS_MAX)
+    if (batch_threads == 0 && factor(W, rad, mid_max_prime(prec)) && mid_prime_of(W, prec, nullptr) > 31 &&
+        W <= 16 * P3E_MID_MAXTH && (size_t)W * 4 * (size_t)prec <= LDS_MAX)
       ok = true;
     if (!ok) ok = factor(W, rad);
     if (!ok) {
@@ -884,39 +1101,41 @@ static bool radix_supported(int r) {
 }
 
 bool retune_pass(int prec, PassDesc &ps, int B, const int *rad, int nrad) {
-  PassArgs &a = ps.args;
-  if (a.fast || a.mid_prime || a.cls == CLS_EMPTY || B < 1 || (B & (B - 1)) || nrad < 0 ||
+  if (ps.args.fast || ps.args.mid_prime > 16 || ps.args.cls == CLS_EMPTY || B < 1 || (B & (B - 1)) || nrad < 0 ||
       nrad > P3E_MAX_RADIX_PASSES)
     return false;
   long prod = 1;
   for (int i = 0; i < nrad; i++) {
-    if (!radix_supported(rad[i])) return false;
-    // the single-buffer path of the batch kernel: radices 2, 3, 4, 5, 8, 16
-    if (a.mid && !mid_base_radix(rad[i])) return false;
+    if (ps.args.mid ? !mid_base_radix(rad[i]) : !radix_supported(rad[i])) return false;
     prod *= rad[i];
   }
-  if (prod != a.L) return false;
-  // passes planned for the batch kernel: no tables in LDS; a single-buffer
-  // pass keeps at most 16 elements per thread of the batch workgroup
-  const int nl = a.pair ? (B + 1) / 2 : B;  // LDS lines of a tile
-  const size_t lds = (a.mid ? 1 : 2) * (size_t)a.lpad * 2 * (size_t)prec * nl;
-  if (lds > LDS_MAX) return false;
-  if (a.mid) {
-    if ((long)nl * a.L > (long)P3E_MID_E * P3E_STEP_THREADS) return false;
-    const int th = std::max(64, ((int)(((long)nl * a.L + P3E_MID_E - 1) / P3E_MID_E) + 63) & ~63);
-    ps.threads = th;
-    a.nthreads = th;
-  }
+  if (prod != ps.args.L) return false;
+  PassDesc t = ps;
+  PassArgs &a = t.args;
   for (int i = 0; i < nrad; i++) a.radix[i] = rad[i];
   a.nrad = nrad;
   set_radix_divs(a);
+  // (a single-buffer pass of the step kernel has no tables in LDS, one with
+  // its own launch does; the other passes here are the step kernel's)
+  if (a.mid) {
+    if (a.pair && B < 2) return false;
+    mid_twiddles(a.radix, a.nrad, t.tw);
+    a.ntw = (int)t.tw.size();
+    a.tw = nullptr;  // the table follows the radix order
+    if (!mid_geometry(prec, t, a.pair ? B / 2 : B, a.tw_in_lds ? 0 : P3E_STEP_THREADS)) return false;
+    ps = t;
+    return true;
+  }
+  const size_t lds = 2 * (size_t)a.lpad * 2 * (size_t)prec * B;
+  if (lds > LDS_MAX) return false;
   a.B = B;
   a.logB = 0;
   while ((1 << a.logB) < B) a.logB++;
   a.ntile_e = (a.ne + B - 1) / B;
   a.div_ntile = make_fastdiv((uint32_t)a.ntile_e);
-  ps.lds_bytes = lds;
-  ps.nblocks = (unsigned int)((unsigned long long)a.ntile_e * (unsigned long long)a.nf);
+  t.lds_bytes = lds;
+  t.nblocks = (unsigned int)((unsigned long long)a.ntile_e * (unsigned long long)a.nf);
+  ps = t;
   return true;
 }
 

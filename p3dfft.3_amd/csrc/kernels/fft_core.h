@@ -17,6 +17,20 @@
 // registers into scratch memory)
 #define P3E_LAMBDA_INL __attribute__((always_inline))
 
+// Hides how a value was computed from the compiler (workgroup-uniform values
+// in scalar registers, per-thread values in vector registers).
+#if defined(__HIP_DEVICE_COMPILE__)
+#define P3E_OPAQUE_S(x)                    \
+  do {                                      \
+    (x) = __builtin_amdgcn_readfirstlane(x); \
+    asm volatile("" : "+s"(x));             \
+  } while (0)
+#define P3E_OPAQUE_V(x) asm volatile("" : "+v"(x))
+#else
+#define P3E_OPAQUE_S(x) ((void)0)
+#define P3E_OPAQUE_V(x) ((void)0)
+#endif
+
 #include "pass_args.h"
 
 namespace p3e {
@@ -41,6 +55,68 @@ template <typename T> P3E_HD P3E_INL cx<T> conj(cx<T> a) { return mk(a.x, -a.y);
 template <typename T> P3E_HD P3E_INL cx<T> rot(cx<T> a, int sgn) {
   // a * (sgn * i)
   return sgn > 0 ? mk(-a.y, a.x) : mk(a.y, -a.x);
+}
+
+// ---------------------------------------------------------------- global accesses
+// Two reals in one load (8 or 16 bytes, aligned to its size).
+template <typename T> struct alignas(2 * sizeof(T)) RealPair {
+  T a, b;
+};
+// Two complex values in one load (16 or 32 bytes, aligned to 16).
+template <typename T> struct alignas(16) CxPair {
+  T ar, ai, br, bi;
+};
+
+// Global accesses of a tile address the array from the tile's first
+// element (a pointer that is the same for the whole workgroup) with 32-bit
+// byte offsets: the planner admits a pass to this path only when every
+// offset within a tile, on both sides, stays below 2^31 bytes.
+template <typename V> P3E_HD P3E_INL V ldg(const char *base, uint32_t off) {
+  return *reinterpret_cast<const V *>(base + off);
+}
+template <typename V> P3E_HD P3E_INL void stg(char *base, uint32_t off, const V &v) {
+  *reinterpret_cast<V *>(base + off) = v;
+}
+// Non-temporal load, for the paired line-order loads (whole lines read
+// once): on a 512^3 FP32 round trip 1.306 -> 1.251 ms (the forward C2C z
+// pass 0.232 -> 0.194 ms).  The same hint on the other loads (unpaired line
+// order, tile order) was slower or no better: 1.266 / 1.254 ms, and the
+// 256-item batch 1.82 -> 2.31 ms with tile-order loads included.
+template <typename V> P3E_HD P3E_INL V ldg_nt(const char *base, uint32_t off) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (sizeof(V) == 8) {
+    const unsigned long long u = __builtin_nontemporal_load(reinterpret_cast<const unsigned long long *>(base + off));
+    return *reinterpret_cast<const V *>(&u);
+  } else if constexpr (sizeof(V) == 16) {
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    const u4 u = __builtin_nontemporal_load(reinterpret_cast<const u4 *>(base + off));
+    return *reinterpret_cast<const V *>(&u);
+  } else {
+    return *reinterpret_cast<const V *>(base + off);
+  }
+#else
+  return *reinterpret_cast<const V *>(base + off);
+#endif
+}
+// Non-temporal store (streaming: the line is not kept in the caches), for
+// line-order stores, which write whole lines; tile-order stores write
+// partial cache lines that the next tile along e completes, and keep stg.
+template <typename V> P3E_HD P3E_INL void stg_nt(char *base, uint32_t off, const V &v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (sizeof(V) == 4) {
+    __builtin_nontemporal_store(*reinterpret_cast<const unsigned *>(&v), reinterpret_cast<unsigned *>(base + off));
+  } else if constexpr (sizeof(V) == 8) {
+    __builtin_nontemporal_store(*reinterpret_cast<const unsigned long long *>(&v),
+                                reinterpret_cast<unsigned long long *>(base + off));
+  } else if constexpr (sizeof(V) == 16) {
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    __builtin_nontemporal_store(*reinterpret_cast<const u4 *>(&v), reinterpret_cast<u4 *>(base + off));
+  } else {
+    *reinterpret_cast<V *>(base + off) = v;
+  }
+#else
+  *reinterpret_cast<V *>(base + off) = v;
+#endif
 }
 
 P3E_HD P3E_INL uint32_t fdiv(uint32_t n, const FastDiv &f) {
@@ -243,14 +319,75 @@ template <typename T, int P, typename Put> P3E_HD P3E_INL void bf_prime(const cx
   }
 }
 
-template <int R> constexpr bool is_base_radix = R == 2 || R == 3 || R == 4 || R == 5 || R == 8 || R == 16;
+template <typename T, int R> P3E_HD P3E_INL void bfly(cx<T> *v, int s);
+
+// Radix A B with A and B coprime, without twiddles (Good-Thomas): with input
+// n = (B n1 + A n2) mod AB and output k = k1 mod A, k2 mod B,
+// w_AB^(n k) = w_A^(n1 k1) w_B^(n2 k2), so A-point DFTs over n1 and B-point
+// DFTs over n2 of the reindexed array.
+template <int A, int B> constexpr int crt(int k1, int k2) {
+  int k = k1;
+  while (k % B != k2) k += A;
+  return k;
+}
+template <typename T, int A, int B> P3E_HD P3E_INL void bf_coprime(cx<T> *v, int s) {
+  cx<T> u[A][B];
+#pragma unroll
+  for (int n2 = 0; n2 < B; n2++) {
+    cx<T> c[A];
+#pragma unroll
+    for (int n1 = 0; n1 < A; n1++) c[n1] = v[(B * n1 + A * n2) % (A * B)];
+    bfly<T, A>(c, s);
+#pragma unroll
+    for (int k1 = 0; k1 < A; k1++) u[k1][n2] = c[k1];
+  }
+#pragma unroll
+  for (int k1 = 0; k1 < A; k1++) {
+    bfly<T, B>(u[k1], s);
+#pragma unroll
+    for (int k2 = 0; k2 < B; k2++) v[crt<A, B>(k1, k2)] = u[k1][k2];
+  }
+}
+
+// radix 9 = 3 x 3: X[k1 + 3 k2] = sum_n2 w3^(n2 k2) w9^(n2 k1) DFT3 over n1 of
+// x[3 n1 + n2]
+template <typename T> P3E_HD P3E_INL void bf9(cx<T> *v, int s) {
+  const T c1 = (T)0.76604444311897803520239265055541668, s1 = (T)0.64278760968653932632264340990726343;   // 2 pi/9
+  const T c2 = (T)0.17364817766693034885171662676931480, s2 = (T)0.98480775301220805936674302458952302;   // 4 pi/9
+  const T c4 = (T)-0.93969262078590838405410927732473147, s4 = (T)0.34202014332566873304409961468225958;  // 8 pi/9
+  const T sg = (T)s;
+  cx<T> u[3][3];
+#pragma unroll
+  for (int n2 = 0; n2 < 3; n2++) {
+    cx<T> c[3] = {v[n2], v[3 + n2], v[6 + n2]};
+    bf3(c, s);
+#pragma unroll
+    for (int k1 = 0; k1 < 3; k1++) u[k1][n2] = c[k1];
+  }
+  u[1][1] = mul(u[1][1], mk(c1, sg * s1));
+  u[1][2] = mul(u[1][2], mk(c2, sg * s2));
+  u[2][1] = mul(u[2][1], mk(c2, sg * s2));
+  u[2][2] = mul(u[2][2], mk(c4, sg * s4));
+#pragma unroll
+  for (int k1 = 0; k1 < 3; k1++) {
+    bf3(u[k1], s);
+#pragma unroll
+    for (int k2 = 0; k2 < 3; k2++) v[k1 + 3 * k2] = u[k1][k2];
+  }
+}
 
 template <typename T, int R> P3E_HD P3E_INL void bfly(cx<T> *v, int s) {
   if constexpr (R == 2) bf2(v);
   else if constexpr (R == 3) bf3(v, s);
   else if constexpr (R == 4) bf4(v, s);
   else if constexpr (R == 5) bf5(v, s);
+  else if constexpr (R == 6) bf_coprime<T, 2, 3>(v, s);
   else if constexpr (R == 8) bf8(v, s);
+  else if constexpr (R == 9) bf9(v, s);
+  else if constexpr (R == 10) bf_coprime<T, 2, 5>(v, s);
+  else if constexpr (R == 12) bf_coprime<T, 4, 3>(v, s);
+  else if constexpr (R == 14) bf_coprime<T, 2, 7>(v, s);
+  else if constexpr (R == 15) bf_coprime<T, 3, 5>(v, s);
   else if constexpr (R == 16) bf16(v, s);
   else bf_prime<T, R>(v, s, [v](int q, cx<T> x) { v[q] = x; });
 }
@@ -424,6 +561,22 @@ template <typename T> P3E_HD P3E_INL T poisson_factor(const PassArgs &p, int kd,
     s += (T)k * (T)k;
   }
   return s > (T)0 ? (T)-1 / s : (T)0;
+}
+
+// Output rule of element k of line j (line j + e0 of the array): the
+// derivative i k, the Poisson operator, the scale.
+template <typename T>
+P3E_HD P3E_INL cx<T> out_rule(const PassArgs &p, cx<T> y, int k, int je, uint32_t f) {
+  if (p.deriv) {
+    T kk;
+    if (k < p.dmid) kk = (T)k;
+    else if (k == p.dmid) kk = (T)0;
+    else kk = (T)(k - p.dg);
+    y = mk(-kk * y.y, kk * y.x);
+  }
+  if (p.spec_op) y = scl(y, poisson_factor<T>(p, k, je, (int)f));
+  if (p.has_scale) y = scl(y, (T)p.scale);
+  return y;
 }
 
 // Phases of one tile of the generic path, shared with the single-buffer

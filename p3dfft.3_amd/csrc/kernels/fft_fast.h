@@ -258,67 +258,6 @@ P3E_HD P3E_INL void c2r_pair_put(const cx<T> *wN, cx<T> *line, int k, cx<T> xk, 
   if (2 * k != M) line[P3E_PAD(M - k)] = add(add(xm, conj(xk)), rot(mul(conj(wN[M - k]), sub(xm, conj(xk))), 1));
 }
 
-// Two reals in one load (8 or 16 bytes, aligned to its size).
-template <typename T> struct alignas(2 * sizeof(T)) RealPair {
-  T a, b;
-};
-// Two complex values in one load (16 or 32 bytes, aligned to 16).
-template <typename T> struct alignas(16) CxPair {
-  T ar, ai, br, bi;
-};
-
-// Global accesses of a tile address the array from the tile's first
-// element (a pointer that is the same for the whole workgroup) with 32-bit
-// byte offsets: the planner admits a pass to this path only when every
-// offset within a tile, on both sides, stays below 2^31 bytes.
-template <typename V> P3E_HD P3E_INL V ldg(const char *base, uint32_t off) {
-  return *reinterpret_cast<const V *>(base + off);
-}
-template <typename V> P3E_HD P3E_INL void stg(char *base, uint32_t off, const V &v) {
-  *reinterpret_cast<V *>(base + off) = v;
-}
-// Non-temporal load, for the paired line-order loads (whole lines read
-// once): on a 512^3 FP32 round trip 1.306 -> 1.251 ms (the forward C2C z
-// pass 0.232 -> 0.194 ms).  The same hint on the other loads (unpaired line
-// order, tile order) was slower or no better: 1.266 / 1.254 ms, and the
-// 256-item batch 1.82 -> 2.31 ms with tile-order loads included.
-template <typename V> P3E_HD P3E_INL V ldg_nt(const char *base, uint32_t off) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  if constexpr (sizeof(V) == 8) {
-    const unsigned long long u = __builtin_nontemporal_load(reinterpret_cast<const unsigned long long *>(base + off));
-    return *reinterpret_cast<const V *>(&u);
-  } else if constexpr (sizeof(V) == 16) {
-    typedef unsigned u4 __attribute__((ext_vector_type(4)));
-    const u4 u = __builtin_nontemporal_load(reinterpret_cast<const u4 *>(base + off));
-    return *reinterpret_cast<const V *>(&u);
-  } else {
-    return *reinterpret_cast<const V *>(base + off);
-  }
-#else
-  return *reinterpret_cast<const V *>(base + off);
-#endif
-}
-// Non-temporal store (streaming: the line is not kept in the caches), for
-// line-order stores, which write whole lines; tile-order stores write
-// partial cache lines that the next tile along e completes, and keep stg.
-template <typename V> P3E_HD P3E_INL void stg_nt(char *base, uint32_t off, const V &v) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  if constexpr (sizeof(V) == 4) {
-    __builtin_nontemporal_store(*reinterpret_cast<const unsigned *>(&v), reinterpret_cast<unsigned *>(base + off));
-  } else if constexpr (sizeof(V) == 8) {
-    __builtin_nontemporal_store(*reinterpret_cast<const unsigned long long *>(&v),
-                                reinterpret_cast<unsigned long long *>(base + off));
-  } else if constexpr (sizeof(V) == 16) {
-    typedef unsigned u4 __attribute__((ext_vector_type(4)));
-    __builtin_nontemporal_store(*reinterpret_cast<const u4 *>(&v), reinterpret_cast<u4 *>(base + off));
-  } else {
-    *reinterpret_cast<V *>(base + off) = v;
-  }
-#else
-  *reinterpret_cast<V *>(base + off) = v;
-#endif
-}
-
 // FULL: the tile has all B lines (nb == B); every entry a thread owns is
 // then inside the tile and the accesses need no bounds checks.
 template <typename T, int M, bool FULL>
@@ -578,22 +517,6 @@ P3E_HD P3E_INL void fast_load(const PassArgs &p, uint32_t f, int e0, int nb, cx<
   TileRegs<T> R;
   fast_fetch<T, M, FULL>(p, f, e0, nb, R, tid, nth);
   fast_put<T, M, FULL>(p, f, e0, nb, R, buf, tid, nth, wN);
-}
-
-// Output rule of element k of line j (line j + e0 of the array): the
-// derivative i k, the Poisson operator, the scale.
-template <typename T>
-P3E_HD P3E_INL cx<T> out_rule(const PassArgs &p, cx<T> y, int k, int je, uint32_t f) {
-  if (p.deriv) {
-    T kk;
-    if (k < p.dmid) kk = (T)k;
-    else if (k == p.dmid) kk = (T)0;
-    else kk = (T)(k - p.dg);
-    y = mk(-kk * y.y, kk * y.x);
-  }
-  if (p.spec_op) y = scl(y, poisson_factor<T>(p, k, je, (int)f));
-  if (p.has_scale) y = scl(y, (T)p.scale);
-  return y;
 }
 
 // R2C output k of a line from the packed spectrum Z:
@@ -1004,11 +927,11 @@ P3E_HD P3E_INL void dct1_tile(const PassArgs &p, uint32_t tile, cx<T> *buf, int 
 // pass needs); the others take part in the barriers.  The branches on the
 // tile being whole and on the DFT sign are uniform over the workgroup.
 // tw, wN: the pass's twiddles and R2C/C2R split factors (in LDS or global
-// memory).
-template <typename T, int M, typename Run, typename Each>
+// memory).  SPLIT: the kernel may be given split DCT-I passes.
+template <typename T, int M, typename Run, typename Each, bool SPLIT = true>
 P3E_HD P3E_INL void fast_tile(const PassArgs &p, uint32_t tile, cx<T> *buf, int nth, Run &run, Each &each,
                               const cx<T> *tw, const cx<T> *wN) {
-  if constexpr (M == 128 || M == 256 || M == 512 || M == 1024) {
+  if constexpr (SPLIT && (M == 128 || M == 256 || M == 512 || M == 1024)) {
     if (p.dct_split) {
       dct1_tile<T, M>(p, tile, buf, nth, run, each, tw);
       return;

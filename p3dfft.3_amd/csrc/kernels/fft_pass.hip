@@ -48,12 +48,38 @@ __global__ void __launch_bounds__(256) pass_kernel(PassArgs p) {
 // Stages of one transform are ordered by launch boundaries: on MI355X each
 // XCD has its own L2, so a kernel boundary is the cheap way to make one
 // stage's output visible to the next stage's tiles on other XCDs.
+// (Batch plans have no split DCT-I: without it these functions stay short
+// enough for plain branches, see step_mid_as.)
 template <typename T, int M>
-__device__ void step_pow2(const PassArgs &p, uint32_t tile, cx<T> *buf) {
+__device__ __noinline__ void step_pow2(const PassArgs &p, uint32_t tile, cx<T> *buf) {
   DevPassRun<T> run{(int)threadIdx.x, p.nthreads};
   DevEach each{(int)threadIdx.x};
-  fast_tile<T, M>(p, tile, buf, p.nthreads, run, each, reinterpret_cast<const cx<T> *>(p.tw),
-                  reinterpret_cast<const cx<T> *>(p.wN));
+  fast_tile<T, M, DevPassRun<T>, DevEach, false>(p, tile, buf, p.nthreads, run, each,
+                                                 reinterpret_cast<const cx<T> *>(p.tw),
+                                                 reinterpret_cast<const cx<T> *>(p.wN));
+}
+
+// A single-buffer pass of the step kernel: no prime radix above 16, and both
+// sides by the load and store phases (batch plans ask for nothing else).  A
+// function per class: one function of all of them is longer than a branch
+// reaches, and the registers the compiler then takes for a long branch are
+// those of the return address, which it had not saved (the kernel never
+// ended).
+template <typename T, int CLS, bool BLUE>
+__device__ __noinline__ void step_mid_as(const PassArgs &p, uint32_t tile, cx<T> *buf) {
+  DevMidRun<T> run{(int)threadIdx.x, p.nthreads};
+  DevEach each{(int)threadIdx.x};
+  mid_tile_as<T, 0, CLS, MID_IN_LDS, MID_OUT_LDS, BLUE>(p, tile, buf, p.nthreads, run, each,
+                                                         reinterpret_cast<const cx<T> *>(p.tw));
+}
+template <typename T, bool BLUE>
+__device__ __forceinline__ void step_mid(const PassArgs &p, uint32_t tile, cx<T> *buf) {
+  switch (p.cls) {
+    case CLS_C2C: step_mid_as<T, CLS_C2C, BLUE>(p, tile, buf); break;
+    case CLS_R2C: step_mid_as<T, CLS_R2C, BLUE>(p, tile, buf); break;
+    case CLS_C2R: step_mid_as<T, CLS_C2R, BLUE>(p, tile, buf); break;
+    default: step_mid_as<T, CLS_R2R, BLUE>(p, tile, buf); break;
+  }
 }
 
 template <typename T>
@@ -84,10 +110,8 @@ __global__ void __launch_bounds__(P3E_STEP_THREADS)
         default: step_pow2<T, 4096>(sp, wi.tile, bufA); break;
       }
     } else if (sp.mid) {
-      DevPassRun<T> run{(int)threadIdx.x, sp.nthreads};
-      DevEach each{(int)threadIdx.x};
-      // batch plans admit no prime radix to the single-buffer path
-      mid_tile<T, 0>(sp, wi.tile, bufA, sp.nthreads, run, each, reinterpret_cast<const cx<T> *>(sp.tw));
+      if (sp.bluestein) step_mid<T, true>(sp, wi.tile, bufA);
+      else step_mid<T, false>(sp, wi.tile, bufA);
     } else {
       cx<T> *bufB = bufA + (size_t)sp.B * sp.lpad;
       run_tile<T>(sp, wi.tile, bufA, bufB, threadIdx.x, blockDim.x, DevBarrier(),
@@ -122,8 +146,8 @@ int launch_mid_pass(const PassArgs *a, int prec, size_t lds_bytes, int threads, 
                     hipStream_t st);  // fft_midk.hip
 int launch_pow2_group(int M, const PassArgs *tab, const uint32_t *start, int n, int prec, size_t lds_bytes,
                       int threads, unsigned int nblocks, hipStream_t st);  // fft_pow2.hip
-int launch_mid_group(const PassArgs *tab, const uint32_t *start, int n, int prec, size_t lds_bytes, int threads,
-                     unsigned int nblocks, hipStream_t st);  // fft_midk.hip
+int launch_mid_group(const PassArgs *a, const PassArgs *tab, const uint32_t *start, int n, int prec, size_t lds_bytes,
+                     int threads, unsigned int nblocks, hipStream_t st);  // fft_midk.hip
 
 }  // namespace p3e
 
@@ -138,8 +162,10 @@ extern "C" int p3e_launch_pass(const p3e::PassArgs *a, int prec, size_t lds_byte
     return p3e::launch_pow2_pass(&b, prec, lds_bytes, threads, nblocks, st);
   }
   if (a->mid) {
-    if (threads < 1 || threads > P3E_MID_THREADS(prec, a->mid_prime)) return (int)hipErrorInvalidValue;
-    return p3e::launch_mid_pass(a, prec, lds_bytes, threads, nblocks, st);
+    if (threads < 1 || threads > P3E_MID_MAXTH || !a->tw_in_lds) return (int)hipErrorInvalidValue;
+    p3e::PassArgs b = *a;
+    p3e::drop_unaligned_pairs(b, prec);
+    return p3e::launch_mid_pass(&b, prec, lds_bytes, threads, nblocks, st);
   }
   if (prec == 8) {
     if (lds_bytes > 65536)
@@ -157,9 +183,10 @@ extern "C" int p3e_launch_pass(const p3e::PassArgs *a, int prec, size_t lds_byte
 
 // One launch of the same pass of n transforms (a batch stage group): kind
 // 1 power-of-two passes of complex length M, kind 2 single-buffer passes
-// without an odd prime radix above 5.  tab (n PassArgs) and start (n + 1
-// workgroup offsets, start[n] = nblocks) are device arrays.
-extern "C" int p3e_launch_group(int kind, int M, const void *tab, const void *start, int n, int prec, size_t lds,
+// without a prime radix above 16.  tab (n PassArgs) and start (n + 1
+// workgroup offsets, start[n] = nblocks) are device arrays; first: a host
+// copy of one of the passes (kind 2: all are of its class and route).
+extern "C" int p3e_launch_group(int kind, int M, const p3e::PassArgs *first, const void *tab, const void *start, int n, int prec, size_t lds,
                                 int threads, unsigned int nblocks, hipStream_t st) {
   if (nblocks == 0 || n <= 0) return 0;
   const p3e::PassArgs *t = (const p3e::PassArgs *)tab;
@@ -169,8 +196,8 @@ extern "C" int p3e_launch_group(int kind, int M, const void *tab, const void *st
     return p3e::launch_pow2_group(M, t, s, n, prec, lds, threads, nblocks, st);
   }
   if (kind == 2) {
-    if (threads < 1 || threads > P3E_MID_THREADS(prec, 0)) return (int)hipErrorInvalidValue;
-    return p3e::launch_mid_group(t, s, n, prec, lds, threads, nblocks, st);
+    if (threads < 1 || threads > P3E_MID_MAXTH) return (int)hipErrorInvalidValue;
+    return p3e::launch_mid_group(first, t, s, n, prec, lds, threads, nblocks, st);
   }
   return (int)hipErrorInvalidValue;
 }

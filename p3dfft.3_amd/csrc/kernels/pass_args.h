@@ -29,7 +29,7 @@ static inline FastDiv make_fastdiv(uint32_t d) {
   return f;
 }
 
-#define P3E_MAX_RADIX_PASSES 24
+#define P3E_MAX_RADIX_PASSES 14
 
 // Load/store orderings of the tile, chosen from the strides so that
 // consecutive threads touch consecutive addresses.
@@ -106,6 +106,13 @@ struct PassArgs {
   // twiddle tables (ntw_a and ntw_b entries) and M/4 + 1 pre-twiddles
   int dct_split;
   int lp2, ntw_a, ntw_b;
+  // single-buffer path: 2^lgl LDS lines at pitch pit (element m of line t at
+  // m pit + t); the first / last radix pass accesses global memory itself;
+  // DCT/DST-II and -III as an N-point FFT; division by nout / 2
+  int lgl, pit;
+  int direct_in, direct_out;
+  int dct_short;
+  FastDiv div_pairs2;
 };
 
 // One entry of a batch work list: tile `tile` of the pass table[pass].
@@ -128,21 +135,16 @@ static inline void drop_unaligned_pairs(PassArgs &a, int prec) {
 
 // elements held in registers per thread by the fast path
 #define P3E_FAST_E 16
-// Single-buffer mixed-radix path: elements of the tile per thread, at most
-#ifndef P3E_MID_E
-#define P3E_MID_E 16
-#endif
-// and its LDS budget per workgroup in bytes (a tile may exceed it up to the
+// Single-buffer mixed-radix path: radix-R butterflies per thread (up to 20
+// complex values in registers; one butterfly of a larger radix)
+constexpr int mid_butterflies(int R) { return R > 10 ? 1 : 20 / R; }
+// its LDS budget per workgroup in bytes (a tile may exceed it up to the
 // 160 KiB of a CU when one line alone does)
 #ifndef P3E_MID_LDS
 #define P3E_MID_LDS (80 * 1024)
 #endif
-// and its largest workgroup for FP32 passes without an odd prime radix
-// (the others, whose butterflies need more registers, use 512)
-#ifndef P3E_MID_MAXTH
+// and its largest workgroup
 #define P3E_MID_MAXTH 512
-#endif
-#define P3E_MID_THREADS(esz, prime) (((esz) == 4 && (prime) == 0) ? P3E_MID_MAXTH : 512)
 // threads per workgroup of the fast path, at most
 #define P3E_FAST_MAX_THREADS 512
 

@@ -48,6 +48,21 @@ template <typename T> struct DevPassRun {
   }
 };
 
+// One radix pass of the single-buffer path: as DevPassRun, with the thread
+// index opaque per pass (fft_mid.h, mid_fft).
+template <typename T> struct DevMidRun {
+  int tid, nth;
+  template <class PS> __device__ __forceinline__ void operator()(PS &ps) const {
+    int td = tid;
+    P3E_OPAQUE_V(td);
+    cx<T> v[PS::SLOTS];
+    if (td < nth) ps.read(td, nth, v);
+    __syncthreads();
+    if (td < nth) ps.write(td, nth, v);
+    __syncthreads();
+  }
+};
+
 // A plain phase of a tile for this thread, then a barrier.
 struct DevEach {
   int tid;
