@@ -14,10 +14,18 @@ namespace p3e {
 // the tile, followed in LDS by the twiddle table (ntw entries) and, for
 // R2C/C2R, the split factors (M + 1 entries): the radix passes and the
 // split/merge read them from LDS instead of issuing global loads (which
-// would compete with the tile's stream for the memory pipeline).  The
-// twiddles are first read after the barrier that ends the load phase; the
-// split factors are read by the C2R load phase itself, so R2C/C2R passes
-// wait at a barrier after copying them.
+// would compete with the tile's stream for the memory pipeline).
+template <typename T> struct FixedStage {
+  static constexpr bool staged = true;
+  TabStage<T> tw, wn;
+  bool has_wn, wait;
+  __device__ __forceinline__ void operator()(int tid) const {
+    tw.store(tid);
+    if (has_wn) wn.store(tid);
+    if (wait) __syncthreads();
+  }
+};
+
 template <typename T, int M>
 __device__ __forceinline__ void pow2_body(const PassArgs &p, uint32_t tile) {
   extern __shared__ unsigned char smem_raw[];
@@ -26,17 +34,32 @@ __device__ __forceinline__ void pow2_body(const PassArgs &p, uint32_t tile) {
   cx<T> *lwn = ltw + p.ntw;
   const cx<T> *gtw = reinterpret_cast<const cx<T> *>(p.tw);
   const cx<T> *gwn = reinterpret_cast<const cx<T> *>(p.wN);
-  const int tid = threadIdx.x, nth = p.nthreads;
-  for (int i = tid; i < p.ntw; i += blockDim.x) ltw[i] = gtw[i];
-  if (p.cls == CLS_R2C || p.cls == CLS_C2R) {
-    for (int i = tid; i <= M; i += blockDim.x) lwn[i] = gwn[i];
-    // the C2R load phase merges (X_k, X_{M-k}) with the split factors, so
-    // they must be in LDS before any thread's load phase
-    __syncthreads();
+  const int tid = threadIdx.x, nth = p.nthreads, step = (int)blockDim.x;
+  const bool r2c = p.cls == CLS_R2C, c2r = p.cls == CLS_C2R;
+  // R2C and the split DCT-I have the longest tables for their tiles: those
+  // are loaded before the tile and written to LDS once the tile's loads are
+  // issued, so that the two latencies overlap (512^3 FP64 R2C pass 0.651 ->
+  // 0.62 ms, 513-point FP32 DCT-I 0.60 -> 0.575 ms; the DCT-I load phase also
+  // reads its pre-twiddles and has to wait for all threads' copies).  The
+  // other passes copy them first, which measured faster (512^3 FP32: C2C y
+  // 0.201 against 0.206 ms, C2R 0.235 against 0.250 ms, which needs the merge
+  // factors before its first value anyway).
+  FixedStage<T> stage{{gtw, ltw, p.ntw, step, {}}, {gwn, lwn, M + 1, step, {}}, r2c, (bool)p.dct_split};
+  if (r2c || p.dct_split) {
+    stage.tw.load(tid);
+    if (r2c) stage.wn.load(tid);
+  } else {
+    for (int i = tid; i < p.ntw; i += step) ltw[i] = gtw[i];
+    if (c2r) {
+      for (int i = tid; i <= M; i += step) lwn[i] = gwn[i];
+      // the C2R load phase merges (X_k, X_{M-k}) with the split factors, so
+      // they must be in LDS before any thread's load phase
+      __syncthreads();
+    }
   }
   DevPassRun<T> run{tid, nth};
   DevEach each{tid};
-  fast_tile<T, M>(p, tile, buf, nth, run, each, ltw, lwn);
+  fast_tile<T, M, DevPassRun<T>, DevEach, true, FixedStage<T>>(p, tile, buf, nth, run, each, ltw, lwn, stage);
 }
 
 template <typename T, int M>

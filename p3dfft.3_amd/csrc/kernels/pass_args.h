@@ -83,9 +83,6 @@ struct PassArgs {
   int mid_prime;     // its odd prime radix 7..47 (0: none); selects the kernel instantiation
   int pair;          // R2C/C2R on the single-buffer path: lines 2t, 2t+1 share LDS line t
                     // as real and imaginary parts (one complex FFT for two real lines)
-  // generic path, radix pass i: division by L / radix[i] (butterflies per
-  // line) and by the pass's input stride Ns = radix[0] ... radix[i-1]
-  FastDiv div_nbf[P3E_MAX_RADIX_PASSES], div_ns[P3E_MAX_RADIX_PASSES];
   // Spectral operator on the output (the Poisson service): 0 none; 1
   // multiply by -1/|k|^2, 0 at k = 0.  The wavenumber of output index i along
   // the pass's axis d, tile axis e and outer axis f (roles r = 0, 1, 2) is i
@@ -113,6 +110,10 @@ struct PassArgs {
   int direct_in, direct_out;
   int dct_short;
   FastDiv div_pairs2;
+  // generic and single-buffer paths, radix pass i: division by the pass's
+  // input stride Ns = radix[0] ... radix[i-1] and (generic) by L / radix[i]
+  // (butterflies per line); last, as only these arrays are long
+  FastDiv div_ns[P3E_MAX_RADIX_PASSES], div_nbf[P3E_MAX_RADIX_PASSES];
 };
 
 // One entry of a batch work list: tile `tile` of the pass table[pass].

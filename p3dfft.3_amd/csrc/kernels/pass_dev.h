@@ -48,6 +48,34 @@ template <typename T> struct DevPassRun {
   }
 };
 
+// Constant tables on their way to LDS: `load` issues a thread's global loads
+// before the tile's own, `store` writes them to LDS after those are issued,
+// so that the two latencies overlap.
+template <typename T> struct TabStage {
+  static constexpr int K = 16 / sizeof(T);  // entries in registers; longer tables copy the rest in store
+  const cx<T> *g;
+  cx<T> *l;
+  int n, step;
+  T v[2 * K];  // (scalars: arrays of cx<double> would live in scratch)
+  __device__ __forceinline__ void load(int tid) {
+#pragma unroll
+    for (int q = 0; q < K; q++) {
+      const int i = tid + q * step;
+      const cx<T> x = g[i < n ? i : 0];
+      v[2 * q] = x.x;
+      v[2 * q + 1] = x.y;
+    }
+  }
+  __device__ __forceinline__ void store(int tid) const {
+#pragma unroll
+    for (int q = 0; q < K; q++) {
+      const int i = tid + q * step;
+      if (i < n) l[i] = mk(v[2 * q], v[2 * q + 1]);
+    }
+    for (int i = tid + K * step; i < n; i += step) l[i] = g[i];
+  }
+};
+
 // One radix pass of the single-buffer path: as DevPassRun, with the thread
 // index opaque per pass (fft_mid.h, mid_fft).
 template <typename T> struct DevMidRun {
