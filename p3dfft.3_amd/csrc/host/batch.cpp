@@ -418,7 +418,7 @@ BatchPlan *batch_create(int prec, int nitems, const OpSpec ops[3], const int ord
   b->lout.assign(out, out + nitems);
   // grouped launches when every pass of every item, planned as a standalone
   // pass, runs on a kernel that has a grouped form; else the step kernel
-  if (plan_items(b, ops, order, 0)) {
+  if (plan_items(b, ops, order, -1)) {
     b->grouped = true;
     for (const PassChain &c : b->chains)
       for (const PassDesc &pd : c.passes)

@@ -716,9 +716,59 @@ static void setup_fast(int prec, const OpSpec &op, PassDesc &ps, int batch_threa
   }
 }
 
+// Which kernel runs a C2C, R2C or C2R pass that has both a compile-time-length
+// kernel and a single-buffer form.  The latter reads and writes tile-order
+// sides without a phase of its own and keeps 128-byte rows for any length;
+// the former has cheaper line-order sides and more lines per workgroup.
+// Times of one pass, compile-time-length / single-buffer kernel (arrays of
+// 40 to 140 MB of n x n x 1024 or n x n x 256 grids; T: tile order, L: line
+// order, load then store):
+//   FP32  C2C TT  1.3-1.6 (72-240 points), 1.04-1.3 (256, 320, 384), 0.8-1.03
+//                 (512); LL 1.0-1.5 (72-240), 0.98 (256), 0.8-0.9 (320, 384);
+//                 TL 0.9-1.05 (256)
+//         R2C TT  1.07-1.45 (72-256), 0.98-1.05 (320-512); LT 1.16-1.57
+//                 (72-240), 0.96 (256), 0.84-0.92 above
+//         C2R TT  1.08-1.64 (72-256), 0.97 (320); TL 0.98-1.37 (72-256), 0.88
+//   FP64  C2C TT  1.2-1.8 (72-384), 1.01-1.15 (512, 640); LL 1.0-1.34 (72-120,
+//                 224, 240), 0.86 (144, 256); TL 1.08-1.2 (64-256), 0.83 (1024)
+//         R2C TT  1.0-1.18 (72-384), 0.96 (512); LT 1.03-1.35 (72-120), below
+//                 1 above
+//         C2R TT  1.02-1.47 (72-512); TL 1.06-1.29 (72-320), 0.99 (384, 512)
+// A pass over less than 8 MiB is bound by the latency of its few workgroups,
+// which the compile-time kernel has less of (128^3 FP32 round trip 0.071
+// against 0.077 ms, 64^3 FP64 0.058 against 0.068 ms).  In grouped launches
+// over a batch the single-buffer kernel wins for C2C at every length of 32 to
+// 128 points (32: 3.2 against 4.0 TB/s, 48: 3.2 / 4.9, 96: 3.3 / 5.4, 120: 4.1
+// / 4.8, 64 and 128: 5.4 / 5.5).
+static bool prefer_mid(int prec, const PassDesc &ps, bool grouped) {
+  const PassArgs &a = ps.args;
+  const int N = a.N;
+  const bool tt = a.load_order == ORD_TILE && a.store_order == ORD_TILE;
+  const bool ll = a.load_order == ORD_LINE && a.store_order == ORD_LINE;
+  const bool odd = !is_pow2(N) && N <= 240;
+  if (grouped) return a.cls == CLS_C2C || odd;
+  if (std::max(ps.in_bytes, ps.out_bytes) < ((size_t)8 << 20)) return false;
+  if (a.cls == CLS_C2C) {
+    if (tt) return prec == 8 || N <= 384;
+    if (prec == 8 && !ll && a.store_order == ORD_LINE) return N <= 256;
+    return odd && !(prec == 8 && N == 144);
+  }
+  if (a.cls == CLS_R2C) {
+    if (tt) return N <= (prec == 8 ? 384 : 256);
+    return odd && (prec == 4 || N <= 120);
+  }
+  if (a.cls == CLS_C2R) {
+    if (tt) return prec == 8 || N <= 256;
+    return prec == 8 ? N <= 320 : N <= 256;
+  }
+  return false;
+}
+
 // ------------------------------------------------------------------ one pass
 bool describe_pass(int prec, int axis, const OpSpec &op, const Layout &lin, const Layout &lout, PassDesc &ps,
                    int batch_threads) {
+  const bool grouped = batch_threads < 0;
+  if (grouped) batch_threads = 0;
   PassArgs &a = ps.args;
   memset(&a, 0, sizeof(a));
   ps.axis = axis;
@@ -921,7 +971,7 @@ bool describe_pass(int prec, int axis, const OpSpec &op, const Layout &lin, cons
   a.dmid = a.dg / 2;
   a.scale = 1.0;
   setup_mid(prec, op, ps, batch_threads);
-  setup_fast(prec, op, ps, batch_threads);
+  if (!(a.mid && batch_threads == 0 && prefer_mid(prec, ps, grouped))) setup_fast(prec, op, ps, batch_threads);
   return true;
 }
 

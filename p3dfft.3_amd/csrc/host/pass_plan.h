@@ -69,7 +69,8 @@ size_t layout_elems(const Layout &l);
 size_t elem_bytes(int prec, int dt);
 
 // batch_threads > 0 plans the pass for the batch (step) kernel, whose
-// workgroups have that many threads; 0 plans it for its own launch.
+// workgroups have that many threads; 0 plans it for its own launch; < 0 for
+// a grouped launch (the same kernels, chosen for many items together).
 bool describe_pass(int prec, int axis, const OpSpec &op, const Layout &lin, const Layout &lout, PassDesc &ps,
                    int batch_threads = 0);
 // ops[a]: operation on logical axis a; order: axes in execution order.
