@@ -395,7 +395,7 @@ static bool mid_geometry(int prec, PassDesc &ps, int nl, int batch_threads) {
   if (out_w + (a.store_order == ORD_LINE ? a.nout * oe : 0) >= G2) return false;
   // (two radix passes at least: one pass accesses one side; a prime radix
   // above 16 writes to LDS only)
-  const bool direct = a.nrad >= 2 && !a.bluestein && batch_threads == 0;
+  const bool direct = a.nrad >= 2 && batch_threads == 0 && (!a.bluestein || a.cls == CLS_C2C);
   a.direct_in = direct && a.load_order == ORD_TILE && (a.cls == CLS_C2C || a.cls == CLS_R2C) &&
                 (double)(a.L / a.radix[0]) * a.is_d * ie + in_w < 2 * G2;
   a.direct_out = direct && a.store_order == ORD_TILE && (a.cls == CLS_C2C || a.cls == CLS_C2R) &&

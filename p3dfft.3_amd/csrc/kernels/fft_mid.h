@@ -31,7 +31,7 @@
 // 8 MiB strides, which only the two-buffer path took, 7.2 -> 1.8-2.2 ms, a
 // 256-point DCT-II pass of 320x256x300 0.218 -> 0.106 ms, the FP64 DST-I pass
 // of 129x255x200 0.117 -> 0.070 ms, an FP64 Bluestein pass of 131 points 0.245
-// -> 0.165 ms.
+// -> 0.131 ms (0.165 through LDS on both sides and a product phase of its own).
 // Shared by the HIP kernels and the host build used by the CPU tests.
 #pragma once
 #include "fft_core.h"
@@ -77,15 +77,21 @@ P3E_HD P3E_INL uint32_t sign_mask(const PassArgs &p) { return p.sign > 0 ? 0x800
 // last one puts its results.  The kernels are instantiated per class and
 // route: a kernel that holds all routes merges their values into one set of
 // registers after each group of loads, and so waits for every group.
-enum MidIn { MID_IN_LDS = 0, MID_IN_CPLX = 1, MID_IN_PAIR = 2 };
-enum MidOut { MID_OUT_LDS = 0, MID_OUT_CPLX = 1, MID_OUT_PAIR = 2, MID_OUT_RULE = 3 };
+// Bluestein (C2C): MID_IN_BLUE multiplies by the chirp and reads no row past
+// the line, MID_OUT_BLUE multiplies by the chirp and drops the rows past it;
+// MID_OUT_HAT ends the first of its two FFTs, with the spectrum product.
+enum MidIn { MID_IN_LDS = 0, MID_IN_CPLX = 1, MID_IN_PAIR = 2, MID_IN_BLUE = 3 };
+enum MidOut {
+  MID_OUT_LDS = 0, MID_OUT_CPLX = 1, MID_OUT_PAIR = 2, MID_OUT_RULE = 3, MID_OUT_BLUE = 4, MID_OUT_HAT = 5
+};
 static inline int mid_in_route(const PassArgs &p) {
   if (!p.direct_in) return MID_IN_LDS;
-  if (p.cls == CLS_C2C) return MID_IN_CPLX;
+  if (p.cls == CLS_C2C) return p.bluestein ? MID_IN_BLUE : MID_IN_CPLX;
   return p.cls == CLS_R2C && p.vec2 ? MID_IN_PAIR : MID_IN_LDS;
 }
 static inline int mid_out_route(const PassArgs &p) {
   if (!p.direct_out) return MID_OUT_LDS;
+  if (p.bluestein) return MID_OUT_BLUE;
   if (p.cls == CLS_C2C) return (p.deriv | p.spec_op | p.has_scale) ? MID_OUT_RULE : MID_OUT_CPLX;
   return p.cls == CLS_C2R && p.vec2s && !p.has_scale ? MID_OUT_PAIR : MID_OUT_LDS;
 }
@@ -130,6 +136,14 @@ template <typename T, int R, int IN, int OUT> struct MPass {
           const long long step = (long long)nbf * p.is_d * CS;
 #pragma unroll
           for (int r = 0; r < R; r++) w[r] = ldg<cx<T>>(gl + r * step, off);
+        } else if constexpr (IN == MID_IN_BLUE) {
+          // rows of the line only: past it, a row that is in the line (the
+          // value is dropped), from a base that is in it too
+          const uint32_t lo = l * (uint32_t)p.is_e * CS, off = (uint32_t)j * (uint32_t)p.is_d * CS + lo;
+          const long long step = (long long)nbf * p.is_d * CS;
+#pragma unroll
+          for (int r = 0; r < R; r++)
+            w[r] = ldg<cx<T>>(r * nbf < p.W ? gl + r * step : gl, j + r * nbf < p.W ? off : lo);
         } else {
           // lines 2l and 2l + 1 of a real array, adjacent in memory
           const uint32_t off = ((uint32_t)j * (uint32_t)p.is_d + 2 * l) * RS;
@@ -158,6 +172,15 @@ template <typename T, int R, int IN, int OUT> struct MPass {
 #pragma unroll
         for (int r = 0; r < R; r++) w[r].y = flip(w[r].y, mask);
       }
+      if constexpr (IN == MID_IN_BLUE) {
+        const cx<T> *ch = reinterpret_cast<const cx<T> *>(p.chirp);
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+          const int n = j + r * nbf;
+          const cx<T> x = mul(w[r], ch[n < p.W ? n : 0]);
+          w[r] = n < p.W ? x : mk((T)0, (T)0);
+        }
+      }
       if (IN == MID_IN_LDS && Ns > 1) {
         k = j - (int)fdiv((uint32_t)j, dns) * Ns;
         const cx<T> *tk = tw + k * (R - 1);
@@ -174,6 +197,26 @@ template <typename T, int R, int IN, int OUT> struct MPass {
           bfly<T, R>(w, -1);
 #pragma unroll
           for (int r = 0; r < R; r++) d[r * step] = w[r];
+        }
+      } else if constexpr (OUT == MID_OUT_HAT) {
+        // last pass of the forward FFT of a convolution: conjugated, so that
+        // the inverse FFT is another forward one
+        const cx<T> *hat = reinterpret_cast<const cx<T> *>(p.chirp_hat);
+        cx<T> *d = t.buf + j * pit + line;
+        bfly<T, R>(w, -1);
+#pragma unroll
+        for (int r = 0; r < R; r++) d[r * nbf * pit] = conj(mul(w[r], hat[j + r * nbf]));
+      } else if constexpr (OUT == MID_OUT_BLUE) {
+        const cx<T> *ch = reinterpret_cast<const cx<T> *>(p.chirp);
+        bfly<T, R>(w, -1);
+        if (line >= t.nl) continue;
+        const uint32_t off = ((uint32_t)j * (uint32_t)p.os_d + (uint32_t)line * (uint32_t)p.os_e) * CS;
+        const long long step = (long long)nbf * p.os_d * CS;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+          const int k = j + r * nbf;
+          if (k >= p.N) continue;
+          stg(gl + r * step, off, out_rule(p, mul(conj(w[r]), ch[k]), k, t.e0 + line, t.f));
         }
       } else {
         // last pass: Ns = L / R, output positions j + r Ns
@@ -200,7 +243,8 @@ template <typename T, int R, int IN, int OUT> struct MPass {
   }
 };
 
-// FFT of length L in place; `run` executes one pass (read half, barrier,
+// FFT of length L in place (Bluestein: both FFTs of the convolution and the
+// spectrum product between them); `run` executes one pass (read half, barrier,
 // write half, barrier).  tw: the twiddles of the passes after the first,
 // pass by pass.  P: the largest prime radix of the instantiation (0: none
 // above 16; 23, 31 and 47 also run the smaller primes above 16, 23 and 31;
@@ -262,11 +306,18 @@ P3E_HD P3E_INL void mid_pass(Run &run, const MidTile<T> &t, int R, int L, int lg
 #undef P3E_MID_CASE
 }
 
-template <typename T, int P, int IN, int OUT, typename Run>
-P3E_HD P3E_INL void mid_fft(Run &run, const MidTile<T> &t, const cx<T> *tw, char *src, char *dst, uint32_t mask) {
+template <typename T, int P, int IN, int OUT, bool BLUE, typename Run>
+P3E_HD P3E_INL void mid_fft(Run &run, const MidTile<T> &t, const cx<T> *tw0, char *src, char *dst, uint32_t mask) {
   const PassArgs &p = t.p;
+  const cx<T> *tw = tw0;
+  const int np = BLUE ? 2 * p.nrad : p.nrad;
   int Ns = 1;
-  for (int i = 0; i < p.nrad; i++) {
+  for (int q = 0; q < np; q++) {
+    const int i = BLUE && q >= p.nrad ? q - p.nrad : q;
+    if (i == 0) {
+      Ns = 1;
+      tw = tw0;
+    }
     const int R = p.radix[i];
     const FastDiv ds = p.div_ns[i];
     int L = p.L, lgl = p.lgl, pit = p.pit;
@@ -276,9 +327,11 @@ P3E_HD P3E_INL void mid_fft(Run &run, const MidTile<T> &t, const cx<T> *tw, char
     P3E_OPAQUE_S(L);
     P3E_OPAQUE_S(lgl);
     P3E_OPAQUE_S(pit);
-    if (IN != MID_IN_LDS && i == 0)
+    if (IN != MID_IN_LDS && q == 0)
       mid_pass<T, P, IN, MID_OUT_LDS>(run, t, R, L, lgl, pit, Ns, ds, tw, src, mask);
-    else if (OUT != MID_OUT_LDS && i == p.nrad - 1)
+    else if (BLUE && q == p.nrad - 1)
+      mid_pass<T, P, MID_IN_LDS, BLUE ? MID_OUT_HAT : MID_OUT_LDS>(run, t, R, L, lgl, pit, Ns, ds, tw, nullptr, 0u);
+    else if (OUT != MID_OUT_LDS && q == np - 1)
       mid_pass<T, P, MID_IN_LDS, OUT>(run, t, R, L, lgl, pit, Ns, ds, tw, dst, mask);
     else
       mid_pass<T, P, MID_IN_LDS, MID_OUT_LDS>(run, t, R, L, lgl, pit, Ns, ds, tw, nullptr, 0u);
@@ -684,25 +737,8 @@ P3E_HD P3E_INL void mid_tile_as(const PassArgs &p, uint32_t tile, cx<T> *buf, in
     });
   }
   char *src = const_cast<char *>(tile_in(t)), *dst = tile_out(t);
-  if constexpr (BLUE) {
-    // Bluestein: forward FFT of the chirped sequence, times the spectrum of
-    // the conjugate chirp, inverse FFT (conjugated; the store conjugates
-    // back and applies the output chirp); one call site for both FFTs
-    for (int h = 0; h < 2; h++) {
-      mid_fft<T, P, IN, OUT>(run, t, tw, src, dst, 0u);
-      if (h == 0)
-        each([&](int tid) P3E_LAMBDA_INL {
-          const cx<T> *hat = reinterpret_cast<const cx<T> *>(p.chirp_hat);
-          if (tid < nth)
-            for (int i = tid; i < p.L << p.lgl; i += nth) {
-              cx<T> *q = buf + (i >> p.lgl) * p.pit + (i & ((1 << p.lgl) - 1));
-              *q = conj(mul(*q, hat[i >> p.lgl]));
-            }
-        });
-    }
-  } else {
-    mid_fft<T, P, IN, OUT>(run, t, tw, src, dst, sign_mask(p));
-  }
+  // Bluestein: the store conjugates back and applies the output chirp
+  mid_fft<T, P, IN, OUT, BLUE>(run, t, tw, src, dst, BLUE ? 0u : sign_mask(p));
   if constexpr (OUT == MID_OUT_LDS)
     each([&](int tid) P3E_LAMBDA_INL {
       if (tid < nth) mid_store<T, CLS, BLUE>(t, tid, nth);
@@ -718,7 +754,13 @@ template <int P, typename F> P3E_HD P3E_INL void mid_dispatch(const PassArgs &p,
   const int in = mid_in_route(p), out = mid_out_route(p);
   if (P <= 16 && p.bluestein) {
     switch (p.cls) {
-      case CLS_C2C: return f(MidC<CLS_C2C>{}, MidC<0>{}, MidC<0>{}, MidC<P <= 16>{});
+      case CLS_C2C:
+        if (in == MID_IN_LDS) {
+          if (out == MID_OUT_LDS) return f(MidC<CLS_C2C>{}, MidC<0>{}, MidC<0>{}, MidC<P <= 16>{});
+          return f(MidC<CLS_C2C>{}, MidC<0>{}, MidC<MID_OUT_BLUE>{}, MidC<P <= 16>{});
+        }
+        if (out == MID_OUT_LDS) return f(MidC<CLS_C2C>{}, MidC<MID_IN_BLUE>{}, MidC<0>{}, MidC<P <= 16>{});
+        return f(MidC<CLS_C2C>{}, MidC<MID_IN_BLUE>{}, MidC<MID_OUT_BLUE>{}, MidC<P <= 16>{});
       case CLS_R2C: return f(MidC<CLS_R2C>{}, MidC<0>{}, MidC<0>{}, MidC<P <= 16>{});
       case CLS_C2R: return f(MidC<CLS_C2R>{}, MidC<0>{}, MidC<0>{}, MidC<P <= 16>{});
       default: return f(MidC<CLS_R2R>{}, MidC<0>{}, MidC<0>{}, MidC<P <= 16>{});

@@ -4,7 +4,7 @@ precision of a case) and on the GPU.
 
 The lengths: one radix pass (11, 16, 17), two (34, 169, 250), three (360,
 1001) and four (1029), composite radices (6, 10, 12, 14, 15), primes above 16
-first (17 * 7, 2 * 47), Bluestein (53, 131), two primes above 16 (323, the
+first (17 * 7, 2 * 47), Bluestein (53 to 997), two primes above 16 (323, the
 generic path); odd line counts leave partial tiles and an unpaired last real
 line.  Tolerance: 8 u log2(points) relative L2 (a radix pass adds a few u of
 relative error per element, log2 of the work length of them at most; the
@@ -21,7 +21,7 @@ import oracle_binding as orc
 # lengths that also have a compile-time kernel, which the planner leaves for
 # this path by order, precision and size: run here with that kernel disabled
 FIXED = [32, 48, 72, 96, 120, 144, 240, 256, 384]
-LENGTHS = [11, 16, 17, 34, 119, 94, 169, 250, 360, 1001, 1029, 53, 131, 323]
+LENGTHS = [11, 16, 17, 34, 119, 94, 169, 250, 360, 1001, 1029, 53, 61, 127, 131, 997, 323]
 # memory orders in and out: both sides along the lines of axis 0, both
 # across, and one of each
 ORDERS = [([0, 1, 2], [0, 1, 2]), ([2, 0, 1], [1, 2, 0]), ([0, 1, 2], [1, 2, 0]), ([1, 2, 0], [0, 2, 1])]
