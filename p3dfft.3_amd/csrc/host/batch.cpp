@@ -280,10 +280,10 @@ static int group_kind(const PassDesc &pd) {
 }
 
 // What the passes of one grouped launch share: the length of a power-of-two
-// kernel, the class and routes of a single-buffer one.
+// kernel; the class, routes and values per thread of a single-buffer one.
 static int group_key(const PassArgs &a) {
   if (a.fast) return a.M;
-  return ((a.cls * 2 + a.bluestein) * 2 + a.direct_in) * 2 + a.direct_out;
+  return (((a.cls * 2 + a.bluestein) * 8 + mid_in_route(a)) * 8 + mid_out_route(a)) * 64 + a.mid_e;
 }
 
 static bool build_groups(BatchPlan *b) {

@@ -275,11 +275,11 @@ static double mid_radix_cost(int R) {
 }
 
 // Threads per LDS line of a radix sequence: every pass has at most
-// mid_butterflies(R) butterflies per thread.
-static int mid_line_threads(int L, const int *rad, int nrad) {
+// mid_butterflies(R, E) butterflies per thread.
+static int mid_line_threads(int L, const int *rad, int nrad, int E) {
   int t = 1;
   for (int i = 0; i < nrad; i++) {
-    const int nb = mid_butterflies(rad[i]);
+    const int nb = mid_butterflies(rad[i], E);
     t = std::max(t, (L / rad[i] + nb - 1) / nb);
   }
   return t;
@@ -287,31 +287,33 @@ static int mid_line_threads(int L, const int *rad, int nrad) {
 
 // Cheapest radix sequence of length L = prime x (a product of base radices):
 // the passes' cost per element, times the threads per line over the ideal
-// L / 20 to the power 1/4 (a sequence whose passes leave many threads idle
-// pays for their registers, not for their work).
-static void mid_search(int L, int rest, int prime, int maxr, std::vector<int> &cur, double cost, double *best,
+// L / E to the power 1/4 (a sequence whose passes leave many threads idle
+// pays for their registers, not for their work).  Of equal ones the last, with
+// the smaller largest radices (16 8 8 for 1024, as on the two-buffer path:
+// the same sums in the same order).
+static void mid_search(int L, int rest, int prime, int E, int maxr, std::vector<int> &cur, double cost, double *best,
                        std::vector<int> *out) {
   if (rest == 1) {
-    const double t = mid_line_threads(L, cur.data(), (int)cur.size());
-    const double c = cost * pow(t * 20.0 / L, 0.25);
-    if (c < *best) {
+    const double t = mid_line_threads(L, cur.data(), (int)cur.size(), E);
+    const double c = cost * pow(t * E / L, 0.25);
+    if (c <= *best) {
       *best = c;
       *out = cur;
     }
     return;
   }
-  if (cost >= *best || cur.size() >= P3E_MAX_RADIX_PASSES) return;
+  if (cost > *best || cur.size() >= P3E_MAX_RADIX_PASSES) return;
   for (int r = std::min(maxr, 16); r >= 2; r--) {
     if (rest % r || !mid_base_radix(r, prime)) continue;
     cur.push_back(r);
-    mid_search(L, rest / r, prime, r, cur, cost + mid_radix_cost(r), best, out);
+    mid_search(L, rest / r, prime, E, r, cur, cost + mid_radix_cost(r), best, out);
     cur.pop_back();
   }
 }
 
-// Radix sequence of work length L (prime: its prime radix above 16 or 0),
-// larger radices first; returns the cost per element.
-static double mid_radices(int L, int prime, std::vector<int> &rad) {
+// Radix sequence of work length L (prime: its prime radix above 16 or 0) at E
+// values per thread, larger radices first; returns the cost per element.
+static double mid_radices(int L, int prime, int E, std::vector<int> &rad) {
   std::vector<int> cur;
   double best = 1e30, c0 = 0;
   rad.clear();
@@ -319,7 +321,7 @@ static double mid_radices(int L, int prime, std::vector<int> &rad) {
     cur.push_back(prime);
     c0 = mid_radix_cost(prime);
   }
-  mid_search(L, prime ? L / prime : L, prime, 16, cur, c0, &best, &rad);
+  mid_search(L, prime ? L / prime : L, prime, E, 16, cur, c0, &best, &rad);
   return best;
 }
 
@@ -373,7 +375,7 @@ static bool mid_geometry(int prec, PassDesc &ps, int nl, int batch_threads) {
   a.B = a.pair ? 2 * nl : nl;
   a.logB = a.pair ? a.lgl + 1 : a.lgl;
   a.lpad = (int)(((long long)a.L * a.pit + a.B - 1) / a.B);
-  const long th = (long)nl * mid_line_threads(a.L, a.radix, a.nrad);
+  const long th = (long)nl * mid_line_threads(a.L, a.radix, a.nrad, a.mid_e);
   if (th > maxth) return false;
   ps.threads = (int)th;
   a.nthreads = (int)th;
@@ -424,12 +426,34 @@ static bool mid_geometry(int prec, PassDesc &ps, int nl, int batch_threads) {
   return true;
 }
 
+// Whether a standalone single-buffer pass t, described with few values per
+// thread at the same tile width, is faster so: twice the wavefronts of half
+// the work.  Time with many values / with few, one pass:
+//   FP64  1.0-1.39 (1024 points LT, LL, TL 1.31-1.39; 300 points R2C and C2R
+//         1.28; LL 192 1.33; DCT-II of 200 points 1.44; Bluestein of 131 points
+//         1.26).  The kernels with a direct side and the derivative or Poisson
+//         rule take 152 VGPRs, three wavefronts a SIMD: one workgroup of more
+//         than 384 threads a CU (512^3 derivative 1.49 -> 1.64 ms; R2C TT of 384
+//         and 512 points 0.92).
+//   FP32  144, 160, 300, 320 points 1.03-1.14 (R2C, C2R), 0.96-1.08 (C2C); 192,
+//         224-256 points 0.97-1.03; 72-120 points 0.80-1.0 and 512-1024 points
+//         0.92-1.0, both bound by throughput; small grids, bound by latency,
+//         1.1-1.2 (104^3).
+// Grouped launches run enough workgroups without it (batch of 256 items of 32
+// to 128 points 1.44 -> 1.49 ms), and a prime radix above 16 sets the registers
+// itself: more threads only wait for its pass (376 points 166 -> 251 us).
+static bool prefer_few(int prec, const PassDesc &t) {
+  const PassArgs &a = t.args;
+  if (prec == 8) return !((a.direct_in || a.direct_out) && t.threads > 384);
+  return std::max(t.in_bytes, t.out_bytes) < ((size_t)8 << 20) || (a.L > 128 && a.L <= 400);
+}
+
 // Switch an already described generic pass to the single-buffer mixed-radix
 // path (fft_mid.h) when its work length is a product of that path's radices
 // (a length with a larger prime factor runs Bluestein's convolution at the
 // cheapest such length of at least 2W - 1).  Other passes stay on the
 // two-buffer generic path.
-static void setup_mid(int prec, const OpSpec &op, PassDesc &ps, int batch_threads) {
+static void setup_mid(int prec, const OpSpec &op, PassDesc &ps, int batch_threads, bool grouped) {
   if (op.cls == CLS_EMPTY || ps.args.nrad < 1) return;
   PassDesc t = ps;
   PassArgs &a = t.args;
@@ -456,56 +480,71 @@ static void setup_mid(int prec, const OpSpec &op, PassDesc &ps, int batch_thread
       for (int q = 0; q < N; q++) tab[q] = expi_pi(inv ? q : -q, 2LL * N);  // e^{+-i pi q / 2N}
     }
   }
-  std::vector<int> rad;
   if (!a.dct_short) {
     prime = a.bluestein ? -1 : mid_prime_of(a.W, prec, &named);
     if (batch_threads > 0 && prime > 0) return;
     if (!a.bluestein && prime < 0) return;
   }
   if (a.bluestein) {
-    // every length up to the next power of two: smallest cost of both FFTs
-    const int lo = 2 * a.W - 1, hi = next_pow2(lo);
-    double best = 1e30;
-    std::vector<int> r;
-    for (int L = lo; L <= hi; L++) {
-      if (mid_prime_of(L, prec, nullptr) != 0) continue;
-      const double c = mid_radices(L, 0, r) * L;
-      if (c < best) {
-        best = c;
-        a.L = L;
-        rad = r;
-      }
-    }
     prime = named = 0;
+    if (op.cls != CLS_R2R) a.zero_fill = 0;
+  }
+  a.mid = 1;
+  a.mid_prime = batch_threads > 0 ? 0 : (prime > 0 ? prime : named);
+  a.pair = op.cls == CLS_R2C || op.cls == CLS_C2R || (op.cls == CLS_R2R && !a.in_cplx && !a.out_cplx);
+  const bool line_both = a.load_order == ORD_LINE && a.store_order == ORD_LINE;
+  const int most = next_pow2(a.pair ? (a.ne + 1) / 2 : a.ne);
+  PassDesc many;
+  int nl_many = 0;
+  for (const int E : {P3E_MID_MANY, P3E_MID_FEW}) {
+    if (E == P3E_MID_FEW && (batch_threads > 0 || grouped || prime > 16)) continue;
+    std::vector<int> rad;
+    a.mid_e = E;
+    if (a.bluestein) {
+      // every length up to the next power of two: smallest cost of both FFTs
+      const int lo = 2 * a.W - 1, hi = next_pow2(lo);
+      double best = 1e30;
+      std::vector<int> r;
+      for (int L = lo; L <= hi; L++) {
+        if (mid_prime_of(L, prec, nullptr) != 0) continue;
+        const double c = mid_radices(L, 0, E, r) * L;
+        if (c < best) {
+          best = c;
+          a.L = L;
+          rad = r;
+        }
+      }
+    } else {
+      mid_radices(a.L, prime, E, rad);
+    }
+    if (rad.empty() || rad.size() > P3E_MAX_RADIX_PASSES) return;
+    a.nrad = (int)rad.size();
+    for (int i = 0; i < a.nrad; i++) a.radix[i] = rad[i];
+    set_radix_divs(a);
+    mid_twiddles(a.radix, a.nrad, t.tw);
+    a.ntw = (int)t.tw.size();
+    // Tile width: rows of 128 bytes of the complex side when a side is tile
+    // order (two of them up to 128 points); half of it when one tile would
+    // not leave room for another workgroup on its CU
+    int nl = std::min((prec == 8 ? 8 : 16) * (!line_both && a.L <= 128 ? 2 : 1), most);
+    while (nl > 1 && (!mid_geometry(prec, t, nl, batch_threads) || t.lds_bytes > P3E_MID_LDS)) nl /= 2;
+    const bool ok = mid_geometry(prec, t, nl, batch_threads);
+    if (E == P3E_MID_MANY) {
+      if (!ok) return;
+      many = t;
+      nl_many = nl;
+    } else if (!ok || nl < nl_many || !prefer_few(prec, t)) {
+      t = many;
+    }
+  }
+  if (a.bluestein) {
     std::vector<cld> b(a.L, cld(0, 0));
     for (int m = 0; m < a.W; m++) b[m] = std::conj(t.chirp[m]);
     for (int m = 1; m < a.W; m++) b[a.L - m] = std::conj(t.chirp[m]);
     host_fft(b);
     for (int m = 0; m < a.L; m++) b[m] /= (long double)a.L;
     t.chirp_hat = b;
-    if (op.cls != CLS_R2R) a.zero_fill = 0;
-  } else {
-    mid_radices(a.L, prime, rad);
   }
-  if (rad.empty() || rad.size() > P3E_MAX_RADIX_PASSES) return;
-  a.nrad = (int)rad.size();
-  for (int i = 0; i < a.nrad; i++) a.radix[i] = rad[i];
-  set_radix_divs(a);
-  mid_twiddles(a.radix, a.nrad, t.tw);
-  a.ntw = (int)t.tw.size();
-  a.mid = 1;
-  a.mid_prime = batch_threads > 0 ? 0 : (prime > 0 ? prime : named);
-  a.pair = op.cls == CLS_R2C || op.cls == CLS_C2R || (op.cls == CLS_R2R && !a.in_cplx && !a.out_cplx);
-  // Tile width: rows of 128 bytes of the complex side when a side is tile
-  // order; half of it when one tile would not leave room for another
-  // workgroup on its CU
-  const bool line_both = a.load_order == ORD_LINE && a.store_order == ORD_LINE;
-  int nl = prec == 8 ? 8 : 16;
-  const int most = next_pow2(a.pair ? (a.ne + 1) / 2 : a.ne);
-  if (!line_both && a.L <= 128) nl *= 2;
-  nl = std::min(nl, most);
-  while (nl > 1 && (!mid_geometry(prec, t, nl, batch_threads) || t.lds_bytes > P3E_MID_LDS)) nl /= 2;
-  if (!mid_geometry(prec, t, nl, batch_threads)) return;
   ps = t;
 }
 
@@ -970,7 +1009,7 @@ bool describe_pass(int prec, int axis, const OpSpec &op, const Layout &lin, cons
   a.dg = (op.cls == CLS_R2C) ? 2 * (nout - 1) : nout;
   a.dmid = a.dg / 2;
   a.scale = 1.0;
-  setup_mid(prec, op, ps, batch_threads);
+  setup_mid(prec, op, ps, batch_threads, grouped);
   if (!(a.mid && batch_threads == 0 && prefer_mid(prec, ps, grouped))) setup_fast(prec, op, ps, batch_threads);
   return true;
 }

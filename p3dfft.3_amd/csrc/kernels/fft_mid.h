@@ -73,34 +73,11 @@ template <typename T> P3E_HD P3E_INL T flip(T y, uint32_t mask) {
 }
 P3E_HD P3E_INL uint32_t sign_mask(const PassArgs &p) { return p.sign > 0 ? 0x80000000u : 0u; }
 
-// Where a kernel's first radix pass takes its operands from and where its
-// last one puts its results.  The kernels are instantiated per class and
-// route: a kernel that holds all routes merges their values into one set of
-// registers after each group of loads, and so waits for every group.
-// Bluestein (C2C): MID_IN_BLUE multiplies by the chirp and reads no row past
-// the line, MID_OUT_BLUE multiplies by the chirp and drops the rows past it;
-// MID_OUT_HAT ends the first of its two FFTs, with the spectrum product.
-enum MidIn { MID_IN_LDS = 0, MID_IN_CPLX = 1, MID_IN_PAIR = 2, MID_IN_BLUE = 3 };
-enum MidOut {
-  MID_OUT_LDS = 0, MID_OUT_CPLX = 1, MID_OUT_PAIR = 2, MID_OUT_RULE = 3, MID_OUT_BLUE = 4, MID_OUT_HAT = 5
-};
-static inline int mid_in_route(const PassArgs &p) {
-  if (!p.direct_in) return MID_IN_LDS;
-  if (p.cls == CLS_C2C) return p.bluestein ? MID_IN_BLUE : MID_IN_CPLX;
-  return p.cls == CLS_R2C && p.vec2 ? MID_IN_PAIR : MID_IN_LDS;
-}
-static inline int mid_out_route(const PassArgs &p) {
-  if (!p.direct_out) return MID_OUT_LDS;
-  if (p.bluestein) return MID_OUT_BLUE;
-  if (p.cls == CLS_C2C) return (p.deriv | p.spec_op | p.has_scale) ? MID_OUT_RULE : MID_OUT_CPLX;
-  return p.cls == CLS_C2R && p.vec2s && !p.has_scale ? MID_OUT_PAIR : MID_OUT_LDS;
-}
-
 // Radix-R pass at input stride Ns of the DFT with sign -1 (a DFT with sign +1
 // is the conjugate of this one of the conjugate; mask: the conjugation at a
 // global side).  IN: MidIn, OUT: MidOut; a prime above 16 writes to LDS only.
-template <typename T, int R, int IN, int OUT> struct MPass {
-  static constexpr int NB = mid_butterflies(R);  // butterflies per thread
+template <typename T, int R, int E, int IN, int OUT> struct MPass {
+  static constexpr int NB = mid_butterflies(R, E);  // butterflies per thread
   static constexpr int SLOTS = NB * R;
   static constexpr uint32_t RS = sizeof(T), CS = 2 * sizeof(T);
   const MidTile<T> &t;
@@ -249,12 +226,12 @@ template <typename T, int R, int IN, int OUT> struct MPass {
 // pass by pass.  P: the largest prime radix of the instantiation (0: none
 // above 16; 23, 31 and 47 also run the smaller primes above 16, 23 and 31;
 // any other prime only itself).
-template <typename T, int P, int IN, int OUT, typename Run>
+template <typename T, int P, int E, int IN, int OUT, typename Run>
 P3E_HD P3E_INL void mid_pass(Run &run, const MidTile<T> &t, int R, int L, int lgl, int pit, int Ns, const FastDiv &dns,
                              const cx<T> *tw, char *gl, uint32_t mask) {
 #define P3E_MID_CASE(RR)                                                   \
   case RR: {                                                               \
-    MPass<T, RR, IN, OUT> ps{t, L, lgl, pit, Ns, dns, tw, gl, mask};       \
+    MPass<T, RR, E, IN, OUT> ps{t, L, lgl, pit, Ns, dns, tw, gl, mask};       \
     run(ps);                                                               \
   } break;
   switch (R) {
@@ -306,7 +283,7 @@ P3E_HD P3E_INL void mid_pass(Run &run, const MidTile<T> &t, int R, int L, int lg
 #undef P3E_MID_CASE
 }
 
-template <typename T, int P, int IN, int OUT, bool BLUE, typename Run>
+template <typename T, int P, int E, int IN, int OUT, bool BLUE, typename Run>
 P3E_HD P3E_INL void mid_fft(Run &run, const MidTile<T> &t, const cx<T> *tw0, char *src, char *dst, uint32_t mask) {
   const PassArgs &p = t.p;
   const cx<T> *tw = tw0;
@@ -328,13 +305,13 @@ P3E_HD P3E_INL void mid_fft(Run &run, const MidTile<T> &t, const cx<T> *tw0, cha
     P3E_OPAQUE_S(lgl);
     P3E_OPAQUE_S(pit);
     if (IN != MID_IN_LDS && q == 0)
-      mid_pass<T, P, IN, MID_OUT_LDS>(run, t, R, L, lgl, pit, Ns, ds, tw, src, mask);
+      mid_pass<T, P, E, IN, MID_OUT_LDS>(run, t, R, L, lgl, pit, Ns, ds, tw, src, mask);
     else if (BLUE && q == p.nrad - 1)
-      mid_pass<T, P, MID_IN_LDS, BLUE ? MID_OUT_HAT : MID_OUT_LDS>(run, t, R, L, lgl, pit, Ns, ds, tw, nullptr, 0u);
+      mid_pass<T, P, E, MID_IN_LDS, BLUE ? MID_OUT_HAT : MID_OUT_LDS>(run, t, R, L, lgl, pit, Ns, ds, tw, nullptr, 0u);
     else if (OUT != MID_OUT_LDS && q == np - 1)
-      mid_pass<T, P, MID_IN_LDS, OUT>(run, t, R, L, lgl, pit, Ns, ds, tw, dst, mask);
+      mid_pass<T, P, E, MID_IN_LDS, OUT>(run, t, R, L, lgl, pit, Ns, ds, tw, dst, mask);
     else
-      mid_pass<T, P, MID_IN_LDS, MID_OUT_LDS>(run, t, R, L, lgl, pit, Ns, ds, tw, nullptr, 0u);
+      mid_pass<T, P, E, MID_IN_LDS, MID_OUT_LDS>(run, t, R, L, lgl, pit, Ns, ds, tw, nullptr, 0u);
     if (Ns > 1) tw += Ns * (R - 1);
     Ns *= R;
   }
@@ -718,7 +695,7 @@ template <typename T, int CLS, bool BLUE> P3E_HD P3E_INL void mid_store(const Mi
 // phase f for the calling thread and ends with a barrier (device), or runs
 // it for every thread in turn (host build).  Only threads tid < nth work;
 // the others take part in the barriers.
-template <typename T, int P, int CLS, int IN, int OUT, bool BLUE, typename Run, typename Each>
+template <typename T, int P, int E, int CLS, int IN, int OUT, bool BLUE, typename Run, typename Each>
 P3E_HD P3E_INL void mid_tile_as(const PassArgs &p, uint32_t tile, cx<T> *buf, int nth, Run &run, Each &each,
                                 const cx<T> *tw) {
   uint32_t f;
@@ -738,7 +715,7 @@ P3E_HD P3E_INL void mid_tile_as(const PassArgs &p, uint32_t tile, cx<T> *buf, in
   }
   char *src = const_cast<char *>(tile_in(t)), *dst = tile_out(t);
   // Bluestein: the store conjugates back and applies the output chirp
-  mid_fft<T, P, IN, OUT, BLUE>(run, t, tw, src, dst, BLUE ? 0u : sign_mask(p));
+  mid_fft<T, P, E, IN, OUT, BLUE>(run, t, tw, src, dst, BLUE ? 0u : sign_mask(p));
   if constexpr (OUT == MID_OUT_LDS)
     each([&](int tid) P3E_LAMBDA_INL {
       if (tid < nth) mid_store<T, CLS, BLUE>(t, tid, nth);
@@ -791,7 +768,11 @@ template <typename T, int P, typename Run, typename Each>
 P3E_HD P3E_INL void mid_tile(const PassArgs &p, uint32_t tile, cx<T> *buf, int nth, Run &run, Each &each,
                              const cx<T> *tw) {
   mid_dispatch<P>(p, [&](auto c, auto in, auto out, auto blue) {
-    mid_tile_as<T, P, c.v, in.v, out.v, blue.v>(p, tile, buf, nth, run, each, tw);
+    if constexpr (P <= 16) {
+      if (p.mid_e == P3E_MID_FEW)
+        return mid_tile_as<T, P, P3E_MID_FEW, c.v, in.v, out.v, blue.v>(p, tile, buf, nth, run, each, tw);
+    }
+    mid_tile_as<T, P, P3E_MID_MANY, c.v, in.v, out.v, blue.v>(p, tile, buf, nth, run, each, tw);
   });
 }
 

@@ -1,11 +1,11 @@
-// Single-buffer mixed-radix kernels without a prime radix above 16, FP64.
+// Single-buffer mixed-radix kernels without a prime radix above 16, FP64 with few values per thread.
 #include "mid_kernels.h"
 
 namespace p3e {
 
-int launch_mid_base_d(const PassArgs *a, const PassArgs *tab, const uint32_t *start, int n, size_t lds_bytes,
-                      int threads, unsigned int nblocks, hipStream_t st) {
-  return launch_mid<double, 0>(a, tab, start, n, lds_bytes, threads, nblocks, st);
+int launch_mid_few_d(const PassArgs *a, const PassArgs *tab, const uint32_t *start, int n, size_t lds_bytes,
+                     int threads, unsigned int nblocks, hipStream_t st) {
+  return launch_mid<double, 0, P3E_MID_FEW>(a, tab, start, n, lds_bytes, threads, nblocks, st);
 }
 
 }  // namespace p3e

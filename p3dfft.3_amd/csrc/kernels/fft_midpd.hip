@@ -4,8 +4,8 @@
 namespace p3e {
 
 int launch_mid_prime_d(const PassArgs *a, size_t lds_bytes, int threads, unsigned int nblocks, hipStream_t st) {
-  if (a->mid_prime <= 23) return launch_mid<double, 23>(a, nullptr, nullptr, 0, lds_bytes, threads, nblocks, st);
-  if (a->mid_prime == 29) return launch_mid<double, 29>(a, nullptr, nullptr, 0, lds_bytes, threads, nblocks, st);
+  if (a->mid_prime <= 23) return launch_mid<double, 23, P3E_MID_MANY>(a, nullptr, nullptr, 0, lds_bytes, threads, nblocks, st);
+  if (a->mid_prime == 29) return launch_mid<double, 29, P3E_MID_MANY>(a, nullptr, nullptr, 0, lds_bytes, threads, nblocks, st);
   return (int)hipErrorInvalidValue;
 }
 

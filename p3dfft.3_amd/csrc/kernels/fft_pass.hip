@@ -69,7 +69,7 @@ template <typename T, int CLS, bool BLUE>
 __device__ __noinline__ void step_mid_as(const PassArgs &p, uint32_t tile, cx<T> *buf) {
   DevMidRun<T> run{(int)threadIdx.x, p.nthreads};
   DevEach each{(int)threadIdx.x};
-  mid_tile_as<T, 0, CLS, MID_IN_LDS, MID_OUT_LDS, BLUE>(p, tile, buf, p.nthreads, run, each,
+  mid_tile_as<T, 0, P3E_MID_MANY, CLS, MID_IN_LDS, MID_OUT_LDS, BLUE>(p, tile, buf, p.nthreads, run, each,
                                                          reinterpret_cast<const cx<T> *>(p.tw));
 }
 template <typename T, bool BLUE>

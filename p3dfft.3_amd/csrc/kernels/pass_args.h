@@ -104,9 +104,11 @@ struct PassArgs {
   int dct_split;
   int lp2, ntw_a, ntw_b;
   // single-buffer path: 2^lgl LDS lines at pitch pit (element m of line t at
-  // m pit + t); the first / last radix pass accesses global memory itself;
+  // m pit + t); values per thread (P3E_MID_FEW or _MANY, which the kernel is
+  // built for); the first / last radix pass accesses global memory itself;
   // DCT/DST-II and -III as an N-point FFT; division by nout / 2
   int lgl, pit;
+  int mid_e;
   int direct_in, direct_out;
   int dct_short;
   FastDiv div_pairs2;
@@ -115,6 +117,29 @@ struct PassArgs {
   // (butterflies per line); last, as only these arrays are long
   FastDiv div_ns[P3E_MAX_RADIX_PASSES], div_nbf[P3E_MAX_RADIX_PASSES];
 };
+
+// Where a single-buffer kernel's first radix pass takes its operands from and where its
+// last one puts its results.  The kernels are instantiated per class and
+// route: a kernel that holds all routes merges their values into one set of
+// registers after each group of loads, and so waits for every group.
+// Bluestein (C2C): MID_IN_BLUE multiplies by the chirp and reads no row past
+// the line, MID_OUT_BLUE multiplies by the chirp and drops the rows past it;
+// MID_OUT_HAT ends the first of its two FFTs, with the spectrum product.
+enum MidIn { MID_IN_LDS = 0, MID_IN_CPLX = 1, MID_IN_PAIR = 2, MID_IN_BLUE = 3 };
+enum MidOut {
+  MID_OUT_LDS = 0, MID_OUT_CPLX = 1, MID_OUT_PAIR = 2, MID_OUT_RULE = 3, MID_OUT_BLUE = 4, MID_OUT_HAT = 5
+};
+static inline int mid_in_route(const PassArgs &p) {
+  if (!p.direct_in) return MID_IN_LDS;
+  if (p.cls == CLS_C2C) return p.bluestein ? MID_IN_BLUE : MID_IN_CPLX;
+  return p.cls == CLS_R2C && p.vec2 ? MID_IN_PAIR : MID_IN_LDS;
+}
+static inline int mid_out_route(const PassArgs &p) {
+  if (!p.direct_out) return MID_OUT_LDS;
+  if (p.bluestein) return MID_OUT_BLUE;
+  if (p.cls == CLS_C2C) return (p.deriv | p.spec_op | p.has_scale) ? MID_OUT_RULE : MID_OUT_CPLX;
+  return p.cls == CLS_C2R && p.vec2s && !p.has_scale ? MID_OUT_PAIR : MID_OUT_LDS;
+}
 
 // One entry of a batch work list: tile `tile` of the pass table[pass].
 struct WorkItem {
@@ -136,9 +161,11 @@ static inline void drop_unaligned_pairs(PassArgs &a, int prec) {
 
 // elements held in registers per thread by the fast path
 #define P3E_FAST_E 16
-// Single-buffer mixed-radix path: radix-R butterflies per thread (up to 20
-// complex values in registers; one butterfly of a larger radix)
-constexpr int mid_butterflies(int R) { return R > 10 ? 1 : 20 / R; }
+// Single-buffer mixed-radix path: complex values in registers per thread
+// (mid_e; one butterfly of a radix above half of it), and radix-R butterflies
+#define P3E_MID_FEW 10
+#define P3E_MID_MANY 20
+constexpr int mid_butterflies(int R, int E) { return 2 * R > E ? 1 : E / R; }
 // its LDS budget per workgroup in bytes (a tile may exceed it up to the
 // 160 KiB of a CU when one line alone does)
 #ifndef P3E_MID_LDS
