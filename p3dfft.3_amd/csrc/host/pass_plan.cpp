@@ -765,17 +765,21 @@ static void setup_fast(int prec, const OpSpec &op, PassDesc &ps, int batch_threa
 //   FP32  C2C TT  1.3-1.6 (72-240 points), 1.04-1.3 (256, 320, 384), 0.8-1.03
 //                 (512); LL 1.0-1.5 (72-240), 0.98 (256), 0.8-0.9 (320, 384);
 //                 TL 0.9-1.05 (256)
-//         R2C TT  1.07-1.45 (72-256), 0.98-1.05 (320-512); LT 1.16-1.57
+//         R2C TT  1.07-1.45 (72-256), 1.01-1.06 (320, 384), 1.02 (512); LT 1.16-1.57
 //                 (72-240), 0.96 (256), 0.84-0.92 above
-//         C2R TT  1.08-1.64 (72-256), 0.97 (320); TL 0.98-1.37 (72-256), 0.88
+//         C2R TT  1.08-1.64 (72-256), 1.01-1.1 (320, 384), 0.88 (512); TL 0.98-1.37 (72-256), 0.88
 //   FP64  C2C TT  1.2-1.8 (72-384), 1.01-1.15 (512, 640); LL 1.0-1.34 (72-120,
 //                 224, 240), 0.86 (144, 256); TL 1.08-1.2 (64-256), 0.83 (1024)
-//         R2C TT  1.0-1.18 (72-384), 0.96 (512); LT 1.03-1.35 (72-120), below
+//         R2C TT  1.0-1.18 (72-384), 0.88 (512); LT 1.03-1.35 (72-120), below
 //                 1 above
 //         C2R TT  1.02-1.47 (72-512); TL 1.06-1.29 (72-320), 0.99 (384, 512)
-// A pass over less than 8 MiB is bound by the latency of its few workgroups,
-// which the compile-time kernel has less of (128^3 FP32 round trip 0.071
-// against 0.077 ms, 64^3 FP64 0.058 against 0.068 ms).  In grouped launches
+// A pass over less than 8 MiB is bound by the latency of its few workgroups:
+// there the ratio is, over grids of 32^3 to 128^3 in FP32 and FP64, for lengths
+// that are no power of two 1.15-1.9 (C2C TT and TL, 48-120 points), 0.94-1.4
+// (C2C LL, R2C LT, C2R TL); 32 and 64 points 1.19-1.21 (C2C TT), 0.92-1.1 (LL),
+// 0.93-1.0 (TL), 1.07-1.15 (R2C LT), 1.02-1.1 (C2R TL); 128 points 1.0 (C2C TT),
+// 0.9-1.05 (LL, TL), 0.93-0.99 (R2C LT), 1.03-1.12 (C2R TL).  Below 256 KiB both
+// take the time of a launch.  In grouped launches
 // over a batch the single-buffer kernel wins for C2C at every length of 32 to
 // 128 points (32: 3.2 against 4.0 TB/s, 48: 3.2 / 4.9, 96: 3.3 / 5.4, 120: 4.1
 // / 4.8, 64 and 128: 5.4 / 5.5).
@@ -786,18 +790,24 @@ static bool prefer_mid(int prec, const PassDesc &ps, bool grouped) {
   const bool ll = a.load_order == ORD_LINE && a.store_order == ORD_LINE;
   const bool odd = !is_pow2(N) && N <= 240;
   if (grouped) return a.cls == CLS_C2C || odd;
-  if (std::max(ps.in_bytes, ps.out_bytes) < ((size_t)8 << 20)) return false;
+  const size_t bytes = std::max(ps.in_bytes, ps.out_bytes);
+  if (bytes < ((size_t)256 << 10)) return false;
+  if (bytes < ((size_t)8 << 20)) {
+    if (odd) return true;
+    if (a.cls == CLS_C2C) return tt && N <= 64;
+    return !tt && (a.cls == CLS_R2C ? N <= 64 : a.cls == CLS_C2R && N <= 128);
+  }
   if (a.cls == CLS_C2C) {
     if (tt) return prec == 8 || N <= 384;
     if (prec == 8 && !ll && a.store_order == ORD_LINE) return N <= 256;
     return odd && !(prec == 8 && N == 144);
   }
   if (a.cls == CLS_R2C) {
-    if (tt) return N <= (prec == 8 ? 384 : 256);
+    if (tt) return N <= 384;
     return odd && (prec == 4 || N <= 120);
   }
   if (a.cls == CLS_C2R) {
-    if (tt) return prec == 8 || N <= 256;
+    if (tt) return prec == 8 || N <= 384;
     return prec == 8 ? N <= 320 : N <= 256;
   }
   return false;
