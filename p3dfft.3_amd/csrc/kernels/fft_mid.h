@@ -29,9 +29,10 @@
 // 360-point C2C pass of 360^3 0.151 -> 0.091 ms (4.1 TB/s), its R2C pass 0.210
 // -> 0.098 ms, a 376-point (8 47) pass 0.350 -> 0.154 ms, a 1024-point pass at
 // 8 MiB strides, which only the two-buffer path took, 7.2 -> 1.8-2.2 ms, a
-// 256-point DCT-II pass of 320x256x300 0.218 -> 0.106 ms, the FP64 DST-I pass
-// of 129x255x200 0.117 -> 0.070 ms, an FP64 Bluestein pass of 131 points 0.245
-// -> 0.131 ms (0.165 through LDS on both sides and a product phase of its own).
+// one 256-point DCT-II call of 320x256x300 0.219 -> 0.113 ms, the FP64 DST-I
+// pass of 129x255x200 0.117 -> 0.070 ms, an FP64 Bluestein pass of 131 points
+// 0.245 -> 0.104 ms (0.165 through LDS on both sides and a product phase of its
+// own, 0.131 with 20 values per thread).
 // Shared by the HIP kernels and the host build used by the CPU tests.
 #pragma once
 #include "fft_core.h"
@@ -577,13 +578,7 @@ template <typename T, int CLS, bool BLUE> P3E_HD P3E_INL cx<T> mid_result(const 
   const cx<T> *post = reinterpret_cast<const cx<T> *>(p.post);
   const int N = p.N;
   if (p.dct_short) {
-    if (p.r2r_kind == REDFT10 || p.r2r_kind == RODFT10) {
-      // Y_k = w^k V_k + conj(w^k) V_{N-k}, w = e^{-i pi / 2N}; DST-II is the
-      // DCT-II of (-1)^n x_n with its outputs reversed
-      const int q = p.r2r_kind == RODFT10 ? N - 1 - k : k;
-      const cx<T> w = post[q];
-      return add(mul(w, mid_get<T, BLUE>(p, line, q)), mul(conj(w), mid_get<T, BLUE>(p, line, q ? N - q : 0)));
-    }
+    // type III (type II: mid_store)
     const cx<T> z = mid_get<T, BLUE>(p, line, (k & 1) ? N - 1 - (k >> 1) : k >> 1);
     return (p.r2r_kind == RODFT01 && (k & 1)) ? mk(-z.x, -z.y) : z;
   }
@@ -665,13 +660,7 @@ template <typename T, int CLS, bool BLUE> P3E_HD P3E_INL void mid_store(const Mi
     }
     return;
   }
-  const int tot = rows * p.nout;
-#pragma unroll 2
-  for (int i = tid; i < tot; i += nth) {
-    int l, k;
-    mid_index(p, along, i, p.nout, p.div_nout, &l, &k);
-    if (l >= nl) continue;
-    cx<T> y = mid_result<T, CLS, BLUE>(p, t.buf + l, k);
+  const auto emit = [&](int l, int k, cx<T> y) P3E_LAMBDA_INL {
     if (p.out_cplx) {
       y = out_rule(p, y, k, t.e0 + l, t.f);
       *reinterpret_cast<cx<T> *>(tout + ((uint32_t)k * osd + (uint32_t)l * (uint32_t)ose) * CS) = y;
@@ -687,6 +676,77 @@ template <typename T, int CLS, bool BLUE> P3E_HD P3E_INL void mid_store(const Mi
         *reinterpret_cast<T *>(q) = y.x;
         if (2 * l + 1 < t.nb) *reinterpret_cast<T *>(q + (size_t)ose * RS) = y.y;
       }
+    }
+  };
+  // groups of G values per thread: the table and LDS reads of a group are all
+  // issued before its stores (which the compiler cannot move reads across; one
+  // 256-point DCT-II call of 320x256x300 FP32 0.121 -> 0.113 ms with both outputs
+  // of a pair in one thread).  The classes without a table are slower so
+  // (300x250x360 FP32 round trip 0.314 -> 0.325 ms)
+  constexpr int G = 16 / sizeof(T);
+  if (CLS == CLS_R2R && p.dct_short && (p.r2r_kind == REDFT10 || p.r2r_kind == RODFT10)) {
+    // a = w^k V_k, b = conj(w^k) V_{N-k}, w = e^{-i pi / 2N}: Y_k = a + b and
+    // Y_{N-k} = i (a - b), both outputs in one thread; DST-II is the DCT-II of
+    // (-1)^n x_n with its outputs reversed
+    const cx<T> *post = reinterpret_cast<const cx<T> *>(p.post);
+    const bool rev = p.r2r_kind == RODFT10;
+    const int H = N / 2 + 1, tot = rows * H;
+    for (int i0 = tid; i0 < tot; i0 += G * nth) {
+      T v[4 * G];
+#pragma unroll
+      for (int u = 0; u < G; u++) {
+        const int i = i0 + u * nth;
+        int l, k;
+        mid_index(p, along, i < tot ? i : 0, H, p.div_pairs, &l, &k);
+        const cx<T> w = post[k];
+        const cx<T> a = mul(w, mid_get<T, BLUE>(p, t.buf + l, k));
+        const cx<T> b = mul(conj(w), mid_get<T, BLUE>(p, t.buf + l, k ? N - k : 0));
+        v[4 * u] = a.x;
+        v[4 * u + 1] = a.y;
+        v[4 * u + 2] = b.x;
+        v[4 * u + 3] = b.y;
+      }
+#pragma unroll
+      for (int u = 0; u < G; u++) {
+        const int i = i0 + u * nth;
+        int l, k;
+        mid_index(p, along, i, H, p.div_pairs, &l, &k);
+        if (!(i < tot && l < nl)) continue;
+        const cx<T> a = mk(v[4 * u], v[4 * u + 1]), b = mk(v[4 * u + 2], v[4 * u + 3]);
+        emit(l, rev ? N - 1 - k : k, add(a, b));
+        if (k && 2 * k != N) emit(l, rev ? k - 1 : N - k, mk(b.y - a.y, a.x - b.x));
+      }
+    }
+    return;
+  }
+  const int tot = rows * p.nout;
+  if constexpr (CLS != CLS_R2R) {
+    // (no table)
+#pragma unroll 2
+    for (int i = tid; i < tot; i += nth) {
+      int l, k;
+      mid_index(p, along, i, p.nout, p.div_nout, &l, &k);
+      if (l < nl) emit(l, k, mid_result<T, CLS, BLUE>(p, t.buf + l, k));
+    }
+    return;
+  }
+  for (int i0 = tid; i0 < tot; i0 += G * nth) {
+    T v[2 * G];
+#pragma unroll
+    for (int u = 0; u < G; u++) {
+      const int i = i0 + u * nth;
+      int l, k;
+      mid_index(p, along, i < tot ? i : 0, p.nout, p.div_nout, &l, &k);
+      const cx<T> y = mid_result<T, CLS, BLUE>(p, t.buf + l, k);
+      v[2 * u] = y.x;
+      v[2 * u + 1] = y.y;
+    }
+#pragma unroll
+    for (int u = 0; u < G; u++) {
+      const int i = i0 + u * nth;
+      int l, k;
+      mid_index(p, along, i, p.nout, p.div_nout, &l, &k);
+      if (i < tot && l < nl) emit(l, k, mk(v[2 * u], v[2 * u + 1]));
     }
   }
 }
